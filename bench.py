@@ -38,8 +38,8 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-# Algorithmic bytes per point of the search kernel (k_knn): the query's FP64
-# xyz (24 B) and grid key (4 B) read once, its covariance record written (one
+# Algorithmic bytes per point of the search (k_knn_lane and the kernels for
+# the rows it leaves): the query's FP64 xyz (24 B) and grid key (4 B) read once, its covariance record written (one
 # 64-byte record: six FP64 entries, the row-flags word and one pad word).
 SEARCH_BYTES_PER_POINT = 92.0
 # HBM traffic of one k_knn launch on the bench workload (4,000,000 points,
@@ -141,7 +141,7 @@ def gpu_leg(args):
                   "traffic_source": (None if traffic is None else
                                      "rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated; k_knn as of "
                                      "commit " + mt["kernel_commit"]),
-                  "kernel": "k_knn (kNN search + FP64 covariance)",
+                  "kernel": "k_knn_lane + k_knn_pair + k_knn_rest (kNN search + FP64 covariance)",
                   "bytes_per_point": SEARCH_BYTES_PER_POINT,
                   "kernel_ms": ms_search},
         roofline_fp64={"bound": "fp64-valu", "achieved": fp64, "peak": FP64_VECTOR_PEAK_TFLOPS,

@@ -160,8 +160,11 @@ void Context::build_batch_index(Batch& b, const std::vector<uint32_t>& fetch)
     launch_tile_colstart(kres, b.dgrids.as<TileGrid>(), T, colbase, b.colstart.as<uint32_t>(),
                          stream);
     b.inv.ensure(N * 4 + 8);
+    b.qord.ensure(N * 4 + 8);
     launch_gather_sorted(vres, xyz_stage.as<double>(), N, b.sx.as<double>(), b.sy.as<double>(),
                          b.sz.as<double>(), b.inv.as<uint32_t>(), stream);
+    launch_tile_query_order(kres, b.dblocks.as<SegBlock>(), static_cast<uint32_t>(b.blocks.size()),
+                            b.dgrids.as<TileGrid>(), b.qord.as<uint32_t>(), stream);
     b.keys = kres;
     b.perm = vres;
     b.idx_valid = true;
@@ -234,7 +237,7 @@ void Context::run_batch(Batch& b, const gf_stage* st, int ns, const int32_t* til
             if (e->q_per_wave > 0) kt.q_per_wave = e->q_per_wave;
         }
     }
-    const int Q = kt.q_per_wave > 0 ? kt.q_per_wave : knn_queries_per_wave(max_k);
+    const int Q = kt.q_per_wave > 0 ? kt.q_per_wave : kQueriesPerWave;
     std::vector<uint32_t> task0(static_cast<size_t>(T) + 1, 0u);
     uint64_t ntasks = 0;
     for (uint32_t t = 0; t < T; ++t) {
@@ -264,6 +267,8 @@ void Context::run_batch(Batch& b, const gf_stage* st, int ns, const int32_t* til
     tt.ntasks = static_cast<uint32_t>(ntasks);
     tt.max_k = max_k;
     tt.q_per_wave = Q;
+    for (const TileInfo& ti : tiles)
+        if (!ti.all_exact) tt.classes |= knn_class_bit(ti.prog.fetch);
 
     KnnOutputs out{};
     if (where == GF_WHERE_DEVICE) {
@@ -278,13 +283,15 @@ void Context::run_batch(Batch& b, const gf_stage* st, int ns, const int32_t* til
         }
         for (int i = 0; i < ns; ++i) out.status[i] = statbuf.as<uint8_t>() + i * N;
     }
-    flagged.ensure(N * 4 + 4);
+    flagged.ensure(N * 12 + 12);
     counters.ensure(64);
     covbuf.ensure(N * 8 * kCovRecord + 8);
     out.flagged = flagged.as<uint32_t>();
+    out.deferred = out.flagged + N;
+    out.heavy = out.deferred + N;
     out.nflagged = counters.as<uint32_t>();
     out.cov = covbuf.as<double>();
-    launch_fill_u32(out.nflagged, 4, 0u, stream);
+    launch_fill_u32(out.nflagged, 8, 0u, stream);
     if (tune.collect_stats) {
         out.counters = reinterpret_cast<unsigned long long*>(counters.as<uint32_t>() + 8);
         launch_fill_u32(counters.as<uint32_t>() + 8, 8, 0u, stream);
@@ -297,6 +304,7 @@ void Context::run_batch(Batch& b, const gf_stage* st, int ns, const int32_t* til
     cv.perm = b.perm;
     cv.keys = b.keys;
     cv.colstart = b.colstart.as<uint32_t>();
+    cv.qord = b.qord.as<uint32_t>();
     cv.n = N;
     cv.g = b.grids.empty() ? GridParams{} : b.grids[0].g;
     FusedProgram prog0 = tiles.empty() ? base : tiles[0].prog;
@@ -398,7 +406,7 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
             if (e->q_per_wave > 0) kt.q_per_wave = e->q_per_wave;
         }
     }
-    const int Q = kt.q_per_wave > 0 ? kt.q_per_wave : knn_queries_per_wave(max_k);
+    const int Q = kt.q_per_wave > 0 ? kt.q_per_wave : kQueriesPerWave;
     // Host-known tables: column bases by capacity, wave tasks.
     std::vector<uint64_t> colbase(T);
     uint64_t centries = 0;
@@ -433,6 +441,7 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
     b.sy.ensure(N * 8 + 8);
     b.sz.ensure(N * 8 + 8);
     b.inv.ensure(N * 4 + 8);
+    b.qord.ensure(N * 4 + 8);
     b.hist.ensure(static_cast<uint64_t>(nb) * 256 * 4 + 8);
     scan_tmp.ensure(scan_scratch_words(static_cast<uint64_t>(nb) * 256 + 1) * 4);
     xyz_stage.ensure(N * 24 + 8);
@@ -456,11 +465,13 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
             out.col[c] = outbuf.as<double>() + static_cast<uint64_t>(c) * N;
         for (int i = 0; i < ns; ++i) out.status[i] = statbuf.as<uint8_t>() + i * N;
     }
-    flagged.ensure(N * 4 + 4);
+    flagged.ensure(N * 12 + 12);
     counters.ensure(128);
     covbuf.ensure(N * 8 * kCovRecord + 8);
     deep_rows.ensure(N * 4 + 4);
     out.flagged = flagged.as<uint32_t>();
+    out.deferred = out.flagged + N;
+    out.heavy = out.deferred + N;
     out.nflagged = counters.as<uint32_t>();
     out.cov = covbuf.as<double>();
     if (tune.collect_stats)
@@ -474,6 +485,8 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
     tt.ntasks = static_cast<uint32_t>(ntasks);
     tt.max_k = max_k;
     tt.q_per_wave = Q;
+    for (const TileInfo& ti : tiles)
+        if (!ti.all_exact) tt.classes |= knn_class_bit(ti.prog.fetch);
     FusedProgram prog0 = tiles[0].prog;
 
     // What the capture depends on.
@@ -482,7 +495,8 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
                                  static_cast<uint64_t>(where), static_cast<uint64_t>(Q),
                                  static_cast<uint64_t>(kt.group_z), static_cast<uint64_t>(kt.ring0),
                                  static_cast<uint64_t>(kt.ring_max),
-                                 static_cast<uint64_t>(kt.small_col), any_exact_tile ? 1u : 0u,
+                                 static_cast<uint64_t>(kt.small_col),
+                                 static_cast<uint64_t>(kt.set_select), any_exact_tile ? 1u : 0u,
                                  tune.collect_stats ? 1u : 0u, tf.size()};
     auto put = [&](const void* p, size_t bytes) {
         for (size_t o = 0; o < bytes; o += 8) {
@@ -501,7 +515,7 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
                           b.dgrids.ptr, b.dbounds.ptr, b.dfetch.ptr, b.dcolbase.ptr, b.dcolpre.ptr,
                           b.dtune.ptr, b.dtiles.ptr, b.dtasks.ptr, b.keys_a.ptr, b.vals_a.ptr,
                           b.keys_b.ptr, b.vals_b.ptr, b.colstart.ptr, b.sx.ptr, b.sy.ptr,
-                          b.sz.ptr, b.inv.ptr, b.hist.ptr, scan_tmp.ptr, xyz_stage.ptr,
+                          b.sz.ptr, b.inv.ptr, b.qord.ptr, b.hist.ptr, scan_tmp.ptr, xyz_stage.ptr,
                           flagged.ptr, counters.ptr, covbuf.ptr};
     put(ptrs, sizeof(ptrs));
     put(out.col, sizeof(out.col));
@@ -559,7 +573,7 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
                               b.dtiles.as<TileInfo>(), stream);
         });
         capture(&b.gexec_b, [&] {
-            launch_fill_u32(out.nflagged, 4, 0u, stream);
+            launch_fill_u32(out.nflagged, 8, 0u, stream);
             if (out.counters) launch_fill_u32(counters.as<uint32_t>() + 8, 8, 0u, stream);
             launch_tile_keys(b.x.as<double>(), b.y.as<double>(), b.z.as<double>(),
                              b.dblocks.as<SegBlock>(), nb, b.dgrids.as<TileGrid>(),
@@ -576,6 +590,8 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
             launch_gather_sorted(vres, xyz_stage.as<double>(), N, b.sx.as<double>(),
                                  b.sy.as<double>(), b.sz.as<double>(), b.inv.as<uint32_t>(),
                                  stream);
+            launch_tile_query_order(kres, b.dblocks.as<SegBlock>(), nb, b.dgrids.as<TileGrid>(),
+                                    b.qord.as<uint32_t>(), stream);
             b.keys = kres;
             b.perm = vres;
             CloudView cv{};
@@ -585,6 +601,7 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
             cv.perm = b.perm;
             cv.keys = b.keys;
             cv.colstart = b.colstart.as<uint32_t>();
+    cv.qord = b.qord.as<uint32_t>();
             cv.n = N;
             launch_knn(cv, prog0, 0, out, kt, stream, &tt);
             if (any_exact_tile) launch_flag_tiles(N, cv.perm, 0, out, tt, stream);
@@ -603,6 +620,7 @@ bool Context::run_batch_graph(Batch& b, int ns, std::vector<TileInfo>& tiles,
     cv.perm = b.perm;
     cv.keys = b.keys;
     cv.colstart = b.colstart.as<uint32_t>();
+    cv.qord = b.qord.as<uint32_t>();
     cv.n = N;
     reset_spans();
     hipEvent_t t_all = mark();

@@ -29,7 +29,6 @@ KnnTuning Context::knn_tuning(const Cloud& cl, uint32_t fetch) const
     if (const TuneEntry* e = tune.entry_for(cloud_rho(cl.bounds, cl.n), fetch)) {
         if (e->group_z > 0) k.group_z = e->group_z - 1;
         if (e->q_per_wave > 0) k.q_per_wave = e->q_per_wave;
-        if (e->knn_waves > 0) k.waves = e->knn_waves;
     }
     return k;
 }
@@ -87,6 +86,8 @@ void Context::build_index(Cloud& cl, uint32_t fetch, double cell)
     cl.inv.ensure(n * 4 + 8);
     launch_gather_sorted(vres, xyz_stage.as<double>(), n, cl.sx.as<double>(),
                          cl.sy.as<double>(), cl.sz.as<double>(), cl.inv.as<uint32_t>(), stream);
+    cl.qord.ensure(n * 4 + 8);
+    launch_query_order(kres, n, g, cl.qord.as<uint32_t>(), stream);
     cl.keys = kres;
     cl.perm = vres;
     cl.g = g;
@@ -112,6 +113,7 @@ CloudView Context::view(const Cloud& cl) const
     v.perm = cl.perm;
     v.keys = cl.keys;
     v.colstart = cl.colstart.as<uint32_t>();
+    v.qord = cl.qord.as<uint32_t>();
     v.n = cl.n;
     v.g = cl.g;
     return v;
@@ -232,13 +234,15 @@ void Context::run_group(Cloud& cl, const gf_stage* st, int ns, double* const* co
         }
         for (int i = 0; i < ns; ++i) out.status[i] = statbuf.as<uint8_t>() + i * n;
     }
-    flagged.ensure(n * 4 + 4);
+    flagged.ensure(n * 12 + 12);
     counters.ensure(64);
     covbuf.ensure(n * 8 * kCovRecord + 8);
     out.flagged = flagged.as<uint32_t>();
+    out.deferred = out.flagged + n;
+    out.heavy = out.deferred + n;
     out.nflagged = counters.as<uint32_t>();
     out.cov = covbuf.as<double>();
-    launch_fill_u32(out.nflagged, 4, 0u, stream);
+    launch_fill_u32(out.nflagged, 8, 0u, stream);
     if (tune.collect_stats) {
         out.counters = reinterpret_cast<unsigned long long*>(counters.as<uint32_t>() + 8);
         launch_fill_u32(counters.as<uint32_t>() + 8, 8, 0u, stream);
@@ -568,11 +572,13 @@ void Context::knn_lists(Cloud& cl, uint32_t k, uint32_t stride, int mode, uint32
     KnnOutputs out{};
     out.ids = ids;
     out.status[0] = status;
-    flagged.ensure(n * 4 + 4);
+    flagged.ensure(n * 12 + 12);
     counters.ensure(128);
     out.flagged = flagged.as<uint32_t>();
+    out.deferred = out.flagged + n;
+    out.heavy = out.deferred + n;
     out.nflagged = counters.as<uint32_t>();
-    launch_fill_u32(out.nflagged, 4, 0u, stream);
+    launch_fill_u32(out.nflagged, 8, 0u, stream);
     const CloudView cv = view(cl);
     const bool early = !all_exact && !cl.kd_valid && tune.kd_overlap_min &&
                        n >= tune.kd_overlap_min;
@@ -759,11 +765,12 @@ void Context::run_group_static(const double* x, const double* y, const double* z
     double* sy = ar.take<double>(n * 8 + 8);
     double* sz = ar.take<double>(n * 8 + 8);
     uint32_t* inv = ar.take<uint32_t>(n * 4 + 8);
+    uint32_t* qord = ar.take<uint32_t>(n * 4 + 8);
     double* xyz = ar.take<double>(n * 24 + 8);
     uint32_t* hist = ar.take<uint32_t>(radix_hist_words(n) * 4);
     uint32_t* scan = ar.take<uint32_t>(
         scan_scratch_words(std::max<uint64_t>(radix_hist_words(n), col_cap)) * 4);
-    uint32_t* flg = ar.take<uint32_t>(n * 4 + 4);
+    uint32_t* flg = ar.take<uint32_t>(n * 12 + 12);
     uint32_t* cnt = ar.take<uint32_t>(64);
     double* cov = ar.take<double>(n * 8 * kCovRecord + 8);
     const uint32_t cap = kd_node_capacity(n) + 1;
@@ -814,6 +821,7 @@ void Context::run_group_static(const double* x, const double* y, const double* z
                       stream);
     launch_colstart(kres, n, g, colstart, stream);
     launch_gather_sorted(vres, xyz, n, sx, sy, sz, inv, stream);
+    launch_query_order(kres, n, g, qord, stream);
     CloudView cv{};
     cv.sx = sx;
     cv.sy = sy;
@@ -821,6 +829,7 @@ void Context::run_group_static(const double* x, const double* y, const double* z
     cv.perm = vres;
     cv.keys = kres;
     cv.colstart = colstart;
+    cv.qord = qord;
     cv.n = n;
     cv.g = g;
 
@@ -828,6 +837,8 @@ void Context::run_group_static(const double* x, const double* y, const double* z
     for (int c = 0; c < ncol_total; ++c) out.col[c] = cols[c];
     for (int i = 0; i < ns; ++i) out.status[i] = status[i];
     out.flagged = flg;
+    out.deferred = flg + n;
+    out.heavy = out.deferred + n;
     out.nflagged = cnt;
     out.cov = cov;
     launch_fill_u32(cnt, 16, 0u, stream);
@@ -1285,9 +1296,11 @@ int gf_optimal_neighborhood(gf_ctx* ctx, gf_cloud* cloud, uint32_t min_k, uint32
         c->outbuf.ensure(n * max_k * 4 + n + 8);
         out.ids = c->outbuf.as<uint32_t>();
         out.status[0] = reinterpret_cast<uint8_t*>(out.ids + n * max_k);
-        c->flagged.ensure(n * 4 + 4);
+        c->flagged.ensure(n * 12 + 12);
         c->counters.ensure(64);
         out.flagged = c->flagged.as<uint32_t>();
+        out.deferred = out.flagged + n;
+    out.heavy = out.deferred + n;
         out.nflagged = c->counters.as<uint32_t>();
         launch_fill_u32(out.nflagged, 8, 0u, c->stream);
         const CloudView cv = c->view(*cl);
@@ -1636,7 +1649,7 @@ int gf_autotune(gf_ctx* ctx, gf_cloud* cloud, const gf_stage* stages, int nstage
         TuneEntry win{};
         try {
             // Coordinate descent: the column-size factor, then the search's
-            // z grouping, queries per wave and waves per workgroup.
+            // queries per wave.
             for (int fi = 0; fi < nfactors; ++fi) {
                 if (!(factors[fi] > 0)) throw Error(GF_ERR_ARG, "factors must be positive");
                 c->tune.forced_factor = factors[fi];
@@ -1648,18 +1661,6 @@ int gf_autotune(gf_ctx* ctx, gf_cloud* cloud, const gf_stage* stages, int nstage
             }
             c->tune.forced_factor = bestf;
             win.cell_factor = bestf;
-            int bestgz = saved.group_z;
-            for (int gz : {0, 1, 2, 3, 4}) {
-                if (gz == saved.group_z) continue;  // measured above
-                c->tune.group_z = gz;
-                const double ms = measure();
-                if (ms < best) {
-                    best = ms;
-                    bestgz = gz;
-                }
-            }
-            c->tune.group_z = bestgz;
-            win.group_z = bestgz + 1;
             const int q0 = saved.q_per_wave;
             int bestq = q0;
             for (int q : {16, 32, 64}) {
@@ -1673,17 +1674,6 @@ int gf_autotune(gf_ctx* ctx, gf_cloud* cloud, const gf_stage* stages, int nstage
             }
             c->tune.q_per_wave = bestq;
             win.q_per_wave = bestq;
-            int bestw = saved.knn_waves;
-            for (int w : {1, 2, 4}) {
-                if (w == saved.knn_waves || (saved.knn_waves == 0 && w == 4)) continue;
-                c->tune.knn_waves = w;
-                const double ms = measure();
-                if (ms < best) {
-                    best = ms;
-                    bestw = w;
-                }
-            }
-            win.knn_waves = bestw;
         } catch (...) {
             c->tune = saved;
             c->timing = timing;

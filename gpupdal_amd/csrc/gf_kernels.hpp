@@ -34,6 +34,9 @@ void launch_radix_sort(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1,
 // read at random instead of three), and the inverse permutation.
 void launch_gather_sorted(const uint32_t* perm, const double* xyz, uint64_t n, double* sx,
                           double* sy, double* sz, uint32_t* inv, hipStream_t s);
+// The order in which the search takes the n sorted positions as queries.
+void launch_query_order(const uint32_t* keys, uint64_t n, const GridParams& g, uint32_t* qord,
+                        hipStream_t s);
 void launch_set_u32(uint32_t* p, uint32_t v, hipStream_t s);
 
 // Tiled batches: segment blocks of <= 4096 points that never cross a tile,
@@ -87,6 +90,9 @@ void launch_seg_radix_sort(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v
                            const SegBlock* blocks, uint32_t nblocks, uint32_t bits,
                            uint32_t* hist, uint32_t* scan_scratch, uint32_t** kres,
                            uint32_t** vres, hipStream_t s);
+// The query order of each tile of a batch (windows never cross a tile).
+void launch_tile_query_order(const uint32_t* keys, const SegBlock* blocks, uint32_t nblocks,
+                             const TileGrid* grids, uint32_t* qord, hipStream_t s);
 void launch_tile_colstart(const uint32_t* keys, const TileGrid* grids, uint32_t T,
                           uint64_t entries, uint32_t* colstart, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
@@ -98,7 +104,13 @@ struct KnnOutputs {
     uint8_t* status[kMaxStages];
     uint32_t* ids;           // neighbor-list mode: n x k (original order)
     uint32_t* flagged;       // sorted indices of tie/incomplete rows
-    uint32_t* nflagged;      // [0] flagged rows, [1] tie rows, [2] incomplete rows
+    uint32_t* nflagged;      // [0] flagged rows, [1] tie rows, [2] incomplete rows,
+                             // [3] rows in deferred, [4] groups in heavy, [7] next heavy
+                             // half group (8 words cleared before a search)
+    uint32_t* deferred;      // sorted indices the lane-per-query search leaves to the
+                             // growing search (up to one per row)
+    uint32_t* heavy;         // query groups whose box holds too many points (up to one
+                             // per row)
     double* cov;             // per sorted row a kCovRecord-double record: the 6 unique
                              // covariance entries, then the row flags (as a uint64)
     unsigned long long* counters; // optional: passes, candidates, merges, queries
@@ -108,10 +120,9 @@ struct KnnTuning {
     int32_t ring0;       // first ring (box half-width in columns)
     int32_t ring_max;    // budget before a row is marked incomplete
     int32_t small_col;   // columns up to this size are taken whole
-    int32_t group_z;     // z cells beyond the first a query group may span
-    int32_t q_per_wave;  // queries per wave (0: by k)
-    int32_t waves;       // waves per workgroup of the single-cloud search (0: 4)
-    int32_t set_select;  // exact-count selection for set neighborhoods (1; 0: sorting)
+    int32_t group_z;     // radius search: z cells beyond the first a query group may span
+    int32_t q_per_wave;  // queries per wave (0: by the number of points)
+    int32_t set_select;  // 1: lane-per-query search; 0: every row by the growing search
 };
 
 struct CloudView {
@@ -121,6 +132,7 @@ struct CloudView {
     const uint32_t* perm;     // sorted position -> original id
     const uint32_t* keys;     // sorted keys
     const uint32_t* colstart; // ncols + 1
+    const uint32_t* qord;     // the search's query order (sorted positions)
     uint64_t n;
     GridParams g;
 };
@@ -175,17 +187,20 @@ struct TileTables {
     const TileInfo* tiles;
     const uint64_t* starts;  // T + 1 tile starts (for row -> tile lookups)
     uint32_t ntiles;
-    // Wave tasks: tile t's rows are cut into runs of q_per_wave queries,
+    // Search tasks: tile t's rows are cut into runs of q_per_wave queries,
     // tasks task0[t] .. task0[t+1]-1 (T + 1 entries; 0 tasks for tiles
     // searched only exactly).
     const uint32_t* task0;
     uint32_t ntasks;
     int32_t max_k;           // largest k over the tiles (LDS sizing)
-    int32_t q_per_wave;      // queries per task
+    int32_t q_per_wave;      // queries per wave
+    uint32_t classes;        // knn_class_bit() of every searched tile's capacity, or-ed
 };
 
-// Queries per wavefront task for a neighborhood of k (LDS lists scale with k).
-inline int knn_queries_per_wave(int max_k) { return max_k <= 32 ? 64 : 32; }
+// Queries per wave of the search.
+constexpr int kQueriesPerWave = 64;
+// The search kernel instance that serves a result capacity, as a bit.
+uint32_t knn_class_bit(int fetch);
 
 // mode 0: neighborhood covariance into out.cov / out.flags (sorted order);
 // mode 1: neighbor lists into out.ids; mode 2: the same, every row with two

@@ -68,10 +68,10 @@ struct Tuning {
     int ring0 = 1;
     int ring_max = 8;
     int small_col = 0;
-    int group_z = 3;             // measured: flat for knn 16, 4% faster search for knn 32
-    int q_per_wave = 0;          // queries per search wave (0: 64 up to k 32, else 32)
-    int knn_waves = 0;           // waves per search workgroup (0: 4)
-    int set_select = 1;          // exact-count selection for set neighborhoods (0: sorting)
+    int group_z = 3;             // radius search: z cells a query group may span
+    int q_per_wave = 0;          // queries per search wave (0: 64)
+    int knn_waves = 0;           // accepted, without effect: the search's workgroups are waves
+    int set_select = 1;          // 1: query-per-lane search; 0: every row by the growing search
     double radius_cell = 0.5;    // radius grids: column edge = radius_cell * radius
     // Exact tree: subtree-per-workgroup threshold (points; 2048-point
     // workgroups, two per CU, measured fastest alone and beside the search).
@@ -188,7 +188,7 @@ struct Cloud {
     double idx_cell = 0.0;       // forced column edge of a radius grid (0: density rule)
     uint64_t idx_tune = 0;
     GridParams g{};
-    DevBuf keys_a, vals_a, keys_b, vals_b, colstart, sx, sy, sz;
+    DevBuf keys_a, vals_a, keys_b, vals_b, colstart, sx, sy, sz, qord;
     uint32_t* keys = nullptr;    // sorted keys (into keys_a/keys_b)
     uint32_t* perm = nullptr;    // sorted position -> original id
     DevBuf inv;                  // original id -> sorted position
@@ -217,7 +217,7 @@ struct Batch {
     std::vector<TileGrid> grids;
     std::vector<double> bounds;          // 6 per tile
     DevBuf dgrids, dbounds, benc, hist;
-    DevBuf keys_a, vals_a, keys_b, vals_b, colstart, sx, sy, sz, inv;
+    DevBuf keys_a, vals_a, keys_b, vals_b, colstart, sx, sy, sz, inv, qord;
     uint32_t* keys = nullptr;
     uint32_t* perm = nullptr;
     uint64_t col_entries = 0;
@@ -325,7 +325,6 @@ struct Context {
         k.small_col = tune.small_col;
         k.group_z = tune.group_z;
         k.q_per_wave = tune.q_per_wave;
-        k.waves = tune.knn_waves;
         k.set_select = tune.set_select;
         return k;
     }

@@ -62,6 +62,11 @@ __device__ __forceinline__ Ent ent_lane(const Ent& e, int src)
 // A value every lane already holds, as a wave-uniform (scalar) value.
 __device__ __forceinline__ int uniform_i32(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+__device__ __forceinline__ uint32_t uniform_u32(uint32_t v)
+{
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
+}
+
 __device__ __forceinline__ double uniform_f64(double v)
 {
     const uint64_t b = static_cast<uint64_t>(__double_as_longlong(v));

@@ -604,6 +604,132 @@ void launch_gather_sorted(const uint32_t* perm, const double* xyz, uint64_t n, d
                        sx, sy, sz, inv);
 }
 
+// --------------------------------------------------------- query order -----
+//
+// The order in which the search takes its queries.  In the index's own order
+// (column, then z) 64 consecutive points of a tall dense place are two or
+// three columns from top to bottom, and the box around them holds several
+// times the points that a compact group's would.  So each window of
+// kOrderWindow sorted positions is sorted by (8 x 8-column tile, block of 8 z
+// cells, Morton order of the cell inside the 8 x 8 x 8 block).  Only the
+// search's grouping of queries depends on it, no result.
+// One workgroup per window, eight keys per thread: a bitonic sort whose
+// short-distance steps stay in registers, the next in cross-lane moves, and
+// only three of the 66 go through LDS.  Keys: tile counted from the window's
+// first (6 bits; further tiles keep the index's order), z block (6 bits),
+// Morton code (9 bits), position in the window (11 bits).
+constexpr uint32_t kOrderWindow = 2048;
+constexpr int kOrderPer = kOrderWindow / 256;
+
+__device__ __forceinline__ uint32_t order_key(uint32_t key, uint32_t bz, uint32_t tile0,
+                                              uint32_t idx)
+{
+    const uint32_t col = key >> bz, z = key & ((1u << bz) - 1u);
+    const uint32_t tile = (col >> 6) - tile0;
+    if (tile >= 63u) return (63u << 26) | idx;
+    // Column bits are x0 y0 x1 y1 x2 y2; z bits go above each pair.
+    uint32_t m = 0;
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+        m |= ((col >> (2 * b) & 3u) | ((z >> b & 1u) << 2)) << (3 * b);
+    return (tile << 26) | (min(z >> 3, 63u) << 20) | (m << 11) | idx;
+}
+
+__device__ __forceinline__ void order_pair(uint32_t& a, uint32_t& b, bool up)
+{
+    const uint32_t lo = min(a, b), hi = max(a, b);
+    a = up ? lo : hi;
+    b = up ? hi : lo;
+}
+
+template <bool kTiled>
+__global__ __launch_bounds__(256) void k_query_order(const uint32_t* __restrict__ keys,
+                                                     uint64_t n, uint32_t bz0,
+                                                     const SegBlock* __restrict__ blocks,
+                                                     const TileGrid* __restrict__ grids,
+                                                     uint32_t* __restrict__ qord)
+{
+    __shared__ uint32_t s_k[kOrderWindow];
+    const uint32_t tid = threadIdx.x;
+    uint64_t base;
+    uint32_t count, bz;
+    if (kTiled) {
+        constexpr uint32_t per = kSegBlockPoints / kOrderWindow;
+        const SegBlock b = blocks[blockIdx.x / per];
+        const uint32_t off = (blockIdx.x % per) * kOrderWindow;
+        if (off >= b.count) return;
+        base = static_cast<uint64_t>(b.begin) + off;
+        count = min(b.count - off, kOrderWindow);
+        bz = grids[b.tile].g.bz;
+    } else {
+        base = static_cast<uint64_t>(blockIdx.x) * kOrderWindow;
+        count = static_cast<uint32_t>(n - base < kOrderWindow ? n - base : kOrderWindow);
+        bz = bz0;
+    }
+    const uint32_t tile0 = (keys[base] >> bz) >> 6;
+    uint32_t v[kOrderPer];
+#pragma unroll
+    for (int r = 0; r < kOrderPer; ++r) {
+        const uint32_t idx = r * 256u + tid;
+        v[r] = idx < count ? order_key(keys[base + idx], bz, tile0, idx) : ~0u;
+    }
+    // Element e = tid * 8 + r.
+#pragma unroll
+    for (uint32_t k = 2; k <= kOrderWindow; k <<= 1) {
+#pragma unroll
+        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+            if (j >= 512u) {  // across waves
+                __syncthreads();
+#pragma unroll
+                for (int r = 0; r < kOrderPer; ++r) s_k[r * 256u + tid] = v[r];
+                __syncthreads();
+                const uint32_t other = tid ^ (j / kOrderPer);
+                const bool up = ((tid * kOrderPer) & k) == 0;
+                const bool lower = ((tid * kOrderPer) & j) == 0;
+#pragma unroll
+                for (int r = 0; r < kOrderPer; ++r) {
+                    const uint32_t o = s_k[r * 256u + other];
+                    v[r] = lower == up ? min(v[r], o) : max(v[r], o);
+                }
+            } else if (j >= static_cast<uint32_t>(kOrderPer)) {  // across lanes
+                const bool up = ((tid * kOrderPer) & k) == 0;
+                const bool lower = ((tid * kOrderPer) & j) == 0;
+#pragma unroll
+                for (int r = 0; r < kOrderPer; ++r) {
+                    const uint32_t o = __shfl_xor(v[r], static_cast<int>(j / kOrderPer));
+                    v[r] = lower == up ? min(v[r], o) : max(v[r], o);
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < kOrderPer; ++r)
+                    if ((r & j) == 0)
+                        order_pair(v[r], v[r | j], ((tid * kOrderPer + r) & k) == 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kOrderPer; ++r) {
+        const uint32_t e = tid * kOrderPer + r;
+        if (e < count) qord[base + e] = static_cast<uint32_t>(base) + (v[r] & (kOrderWindow - 1u));
+    }
+}
+
+void launch_query_order(const uint32_t* keys, uint64_t n, const GridParams& g, uint32_t* qord,
+                        hipStream_t s)
+{
+    if (!n) return;
+    hipLaunchKernelGGL(k_query_order<false>, dim3(div_up(n, kOrderWindow)), dim3(256), 0, s, keys,
+                       n, g.bz, nullptr, nullptr, qord);
+}
+
+void launch_tile_query_order(const uint32_t* keys, const SegBlock* blocks, uint32_t nblocks,
+                             const TileGrid* grids, uint32_t* qord, hipStream_t s)
+{
+    if (!nblocks) return;
+    hipLaunchKernelGGL(k_query_order<true>, dim3(nblocks * (kSegBlockPoints / kOrderWindow)),
+                       dim3(256), 0, s, keys, 0, 0u, blocks, grids, qord);
+}
+
 // Writes colstart[ncols] = n after the exclusive scan of the column counts.
 __global__ void k_set_u32(uint32_t* p, uint32_t v) { *p = v; }
 

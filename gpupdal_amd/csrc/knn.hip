@@ -7,31 +7,24 @@
 // (src/index/SpatialIndexKernels.cu:716-1086, 1716-1769;
 // src/stages/NeighborhoodKernels.cu:67-119, 422-485).
 //
-// Work split.  A wave owns Q consecutive sorted points (queries).  Sorted
-// order is (column, z cell), so consecutive queries form groups that share a
-// column and a short z range; every query of a group has the same candidate
-// box (the 3x3 columns around it, z cells [first-1, last+1]).  The wave loads
-// the box once -- column starts, z-window bounds, the candidates' FP64
-// coordinates and ids -- into registers (up to 256 candidates, 4 per lane),
-// then for each query of the group computes the FP64 squared distances
-// exactly as KD3Index does (d0*d0 + d1*d1 + d2*d2, left to right, no FMA)
-// and selects the fetch+1 smallest (d2, point id) pairs:  a bisection on d2
-// counted with ballots finds a threshold that keeps between fetch+1 and 64
-// candidates, which are compacted through LDS and sorted once by a bitonic
-// network across the lanes.
+// Two kernels share the work: k_knn_lane searches up to 64 consecutive sorted
+// queries per wave, one per lane, over one shared candidate box (see there);
+// k_knn_rest searches the few rows that leaves, one per wave, with a box that
+// grows around the row's own cell.  Both find the fetch + 1 smallest (d2,
+// point id) pairs with the FP64 squared distances KD3Index computes (d0*d0 +
+// d1*d1 + d2*d2, left to right, no FMA).
 //
 // Certification.  A query's list is exact when its fetch-th distance is below
-// the distance from the query to the nearest face of the examined box that
-// borders unexamined grid cells (minus a rounding margin).  Otherwise the
-// query alone is searched again with a growing box (streaming candidates
-// through sort-and-merge) up to a budget; a query still uncertified is
-// flagged incomplete.  Rows whose fetch-th and (fetch+1)-th distances are
-// equal have a boundary tie, which KD3Index breaks by tree visit order rather
-// than by index; they are flagged for the exact KD3 search.
+// the distance from the query to the nearest face of the examined region
+// (minus a rounding margin).  A query still uncertified when the growing
+// box reaches the budget is flagged incomplete.  Rows whose fetch-th and
+// (fetch+1)-th distances are equal have a boundary tie, which KD3Index breaks
+// by tree visit order rather than by index; both kinds go to the exact KD3
+// search.
 //
-// Covariance.  Each query's kept list is parked in LDS; after the wave's
-// queries every lane takes one of them and forms its FP64 covariance
-// (two-pass mean), written in sorted order for the eigen/feature kernel.
+// Covariance.  A row's FP64 covariance (two-pass mean) is formed by one lane
+// from the kept list in (d2, id) order, the same sums in the same order in
+// both kernels, and written in sorted order for the eigen/feature kernel.
 #include "gf_eigen.hpp"
 #include "gf_internal.hpp"
 #include "gf_kernels.hpp"
@@ -41,18 +34,15 @@ namespace gf {
 
 namespace {
 
-// Waves per workgroup.  One cloud: four, so the tree built beside the search
-// finds the slots a workgroup's early waves leave idle until its last wave
-// ends.  Tiles of a batch: one; a wave's slot and LDS free as soon as it ends
-// (measured: the batch's search 6% faster, the step 7% faster).
-// Waves per workgroup: one for the tiled (batch) search, 1, 2 or 4 (tuning
-// "knn_waves", default 4) for a single cloud.
-constexpr int kKnnWavesDefault = 4;
-constexpr int kRegBatches = 4;
+constexpr uint32_t kLaneSmall = 8;     // columns of up to this many points are taken whole
+constexpr int kRegBatches = 8;   // candidates of one row in registers, 64 a batch
 constexpr uint32_t kRegCand = kRegBatches * 64;
-// Per-wave LDS scratch: 64 compacted entries (16 B), 64 ranked entries, and a
-// 64-entry list of queries left for the growing search.
-constexpr int kScratchWords = 256 + 256 + 64;
+constexpr int kGroupBatches = 4; // the same for the box a group of rows shares
+constexpr uint32_t kGroupCand = kGroupBatches * 64;
+constexpr int kRadBatches = 4;   // the same for a radius group's shared box
+constexpr uint32_t kRadCand = kRadBatches * 64;
+// Per-wave LDS scratch: 64 compacted entries (16 B) and 64 ranked entries.
+constexpr int kScratchWords = 256 + 256;
 
 // First positions in a[lo, hi) (sorted ascending) of keys >= k0 and of keys
 // >= k1 (k0 <= k1): two binary searches advanced together, so that their
@@ -104,9 +94,12 @@ struct KnnArgs {
     int32_t lds_stride;
     double margin;
     const TileInfo* tiles;   // tiled search only
+    const uint64_t* starts;  // tiled: first row of each tile (ntiles + 1)
     const uint32_t* task0;   // tiled: per-tile first task (ntiles + 1)
     uint32_t ntasks;
     uint32_t ntiles;
+    int32_t fetch_lo, fetch_hi;  // tiled: the result capacities this launch serves
+    int32_t all_rows;        // k_knn_rest: every row instead of out.deferred
 };
 
 // What a wavefront needs of its cloud or tile: the grid, the column starts,
@@ -153,9 +146,11 @@ __device__ __forceinline__ bool certified(const WaveGrid& wg, const Box& b, cons
 
 // Column ranges of a box, one column per lane (box columns must be <= 64):
 // lo / len of the column's sorted points restricted to z cells [z0, z1]
-// (whole columns when the box spans every z cell or the column is small).
+// (whole columns when the box spans every z cell or the column holds at most
+// `small` points).
 __device__ __forceinline__ void box_ranges(const KnnArgs& a, const WaveGrid& wg, const Box& b,
-                                           int cb, int lane, uint32_t& lo, uint32_t& len)
+                                           int cb, int lane, uint32_t small, uint32_t& lo,
+                                           uint32_t& len)
 {
     const CloudView& cv = a.cv;
     const GridParams& g = wg.g;
@@ -172,13 +167,59 @@ __device__ __forceinline__ void box_ranges(const KnnArgs& a, const WaveGrid& wg,
     const bool zfull = b.z0 <= 0 && b.z1 >= static_cast<int>(g.gz) - 1;
     const uint32_t col = column_index(g, cx, cy);
     uint32_t b0 = wg.colstart[col], b1 = wg.colstart[col + 1];
-    if (!zfull && b1 - b0 > static_cast<uint32_t>(a.tune.small_col)) {
+    if (!zfull && b1 - b0 > small) {
         const uint32_t klo = (col << g.bz) + static_cast<uint32_t>(max(b.z0, 0));
         const uint32_t khi = (col << g.bz) + static_cast<uint32_t>(min(b.z1, static_cast<int>(g.gz) - 1) + 1);
         lower_bound2_u32(cv.keys, b0, b1, klo, khi, b0, b1);
     }
     lo = b0;
     len = b1 - b0;
+}
+
+// The same for a box of ncb <= kCols * 64 columns inside the grid, kCols
+// columns per lane, their loads side by side: column starts first, then the
+// z windows of columns of more than kLaneSmall points, all searched together.
+template <int kCols>
+__device__ __forceinline__ void box_columns(const KnnArgs& a, const WaveGrid& wg, const Box& b,
+                                            int ncb, int lane, uint32_t (&lo)[kCols],
+                                            uint32_t (&len)[kCols])
+{
+    const GridParams& g = wg.g;
+    const int w = b.x1 - b.x0 + 1;
+    const float inv_w = 1.0f / static_cast<float>(w);
+    const bool zfull = b.z0 <= 0 && b.z1 >= static_cast<int>(g.gz) - 1;
+    uint32_t col[kCols];
+#pragma unroll
+    for (int i = 0; i < kCols; ++i) {
+        lo[i] = len[i] = col[i] = 0;
+        const int ci = i * 64 + lane;
+        if (ci < ncb) {
+            // ci / w: ci < 2^10, so the rounded quotient is exact
+            const int cy = static_cast<int>((static_cast<float>(ci) + 0.5f) * inv_w);
+            col[i] = column_index(g, static_cast<uint32_t>(b.x0 + ci - cy * w),
+                                  static_cast<uint32_t>(b.y0 + cy));
+            lo[i] = wg.colstart[col[i]];
+            len[i] = wg.colstart[col[i] + 1];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kCols; ++i) len[i] -= lo[i];
+    if (zfull) return;
+    bool tall = false;
+#pragma unroll
+    for (int i = 0; i < kCols; ++i) tall |= len[i] > kLaneSmall;
+    if (!__ballot(tall)) return;
+#pragma unroll
+    for (int i = 0; i < kCols; ++i) {
+        if (len[i] > kLaneSmall) {
+            const uint32_t klo = (col[i] << g.bz) + static_cast<uint32_t>(b.z0);
+            const uint32_t khi = (col[i] << g.bz) + static_cast<uint32_t>(b.z1 + 1);
+            uint32_t r0, r1;
+            lower_bound2_u32(a.cv.keys, lo[i], lo[i] + len[i], klo, khi, r0, r1);
+            lo[i] = r0;
+            len[i] = r1 - r0;
+        }
+    }
 }
 
 // Sorted position of candidate t of the packed ranges: the lane whose range
@@ -239,13 +280,10 @@ __device__ __forceinline__ uint32_t rank_step(const uint4 e, uint64_t d, uint32_
            (static_cast<uint32_t>(od == d) & static_cast<uint32_t>(e.z < id));
 }
 
-// Selection over at most 256 candidate entries held in registers (4 per
-// lane).  First a threshold E with need <= #{d2 <= E} <= cap (need = fetch +
-// 1, so the (fetch+1)-th entry that decides ties is kept), each trial counted
-// exactly by ballots: the caller's estimate (the previous query's need-th d2)
-// first, then two steps that interpolate the count linearly in d2 (points on
-// a surface: count grows with the area, i.e. with d2) inside the bracket, then
-// bisection.  The survivors are compacted into LDS and ranked: each
+// Selection over at most kRegCand candidate entries held in registers.  First a threshold E with need <= #{d2 <= E} <= cap (need = fetch +
+// 1, so the (fetch+1)-th entry that decides ties is kept), by bisection on
+// d2, each trial counted exactly by ballots.  The survivors are compacted into
+// LDS and ranked: each
 // lane counts the survivors that precede its own entry in (d2, id) order,
 // reading them as LDS broadcasts, and stores itself at that rank.  Every
 // candidate with d2 equal to the boundary distance is below E, so the first
@@ -255,9 +293,12 @@ __device__ __forceinline__ uint32_t rank_step(const uint4 e, uint64_t d, uint32_
 //
 // The lane's candidate of register batch b is (cd[b], cid[b], cj[b]): squared
 // distance bits (kInfD: none), point id and sorted position.
-__device__ __forceinline__ void select_entries(const uint64_t (&cd)[kRegBatches],
-                                               const uint32_t (&cid)[kRegBatches],
-                                               const uint32_t (&cj)[kRegBatches], uint32_t tot,
+// (hint: a threshold to try first, as the previous query's need-th distance;
+// INFINITY for none.)
+template <int NB>
+__device__ __forceinline__ void select_entries(const uint64_t (&cd)[NB],
+                                               const uint32_t (&cid)[NB],
+                                               const uint32_t (&cj)[NB], uint32_t tot,
                                                int fetch, int lane, uint32_t* scratch,
                                                double hint, Ent& best, uint64_t* cnt)
 {
@@ -272,13 +313,13 @@ __device__ __forceinline__ void select_entries(const uint64_t (&cd)[kRegBatches]
         auto count_le = [&](double t) {
             uint32_t k = 0;
 #pragma unroll
-            for (int b = 0; b < kRegBatches; ++b)
+            for (int b = 0; b < NB; ++b)
                 if (static_cast<uint32_t>(b) < nbat)
                     k += __popcll(__ballot(cd[b] != kInfD && bits_d2(cd[b]) <= t));
             return k;
         };
-        double lo_e = 0.0, hi_e = INFINITY;
         ok = false;
+        double lo_e = 0.0, hi_e = INFINITY;
         if (hint < INFINITY) {
             const uint32_t k = count_le(hint);
             if (k >= need && k <= cap) {
@@ -293,7 +334,7 @@ __device__ __forceinline__ void select_entries(const uint64_t (&cd)[kRegBatches]
         if (!ok && hi_e == INFINITY) {
             double mx = 0.0;
 #pragma unroll
-            for (int b = 0; b < kRegBatches; ++b)
+            for (int b = 0; b < NB; ++b)
                 if (static_cast<uint32_t>(b) < nbat && cd[b] != kInfD) mx = fmax(mx, bits_d2(cd[b]));
 #pragma unroll
             for (int m = 32; m > 0; m >>= 1) mx = fmax(mx, __shfl_xor(mx, m));
@@ -318,7 +359,7 @@ __device__ __forceinline__ void select_entries(const uint64_t (&cd)[kRegBatches]
         uint32_t S = 0;
         const uint32_t nbat_s = (tot + 63u) >> 6;
 #pragma unroll
-        for (int b = 0; b < kRegBatches; ++b) {
+        for (int b = 0; b < NB; ++b) {
             if (static_cast<uint32_t>(b) >= nbat_s) break;
             const bool s = cd[b] != kInfD && bits_d2(cd[b]) <= E;
             const uint64_t m = __ballot(s);
@@ -372,7 +413,7 @@ __device__ __forceinline__ void select_entries(const uint64_t (&cd)[kRegBatches]
     }
     best = ent_inf();
 #pragma unroll
-    for (int b = 0; b < kRegBatches; ++b) {
+    for (int b = 0; b < NB; ++b) {
         if (static_cast<uint32_t>(b * 64) >= tot) break;
         Ent c = cd[b] != kInfD ? Ent{cd[b], cid[b], cj[b]} : ent_inf();
         bitonic_sort64(c, lane);
@@ -384,12 +425,12 @@ __device__ __forceinline__ void select_entries(const uint64_t (&cd)[kRegBatches]
 // Candidates whose d2 bits are <= t (below t when kStrict); kInfD entries
 // never count.  Non-negative doubles order as their bit patterns.
 template <bool kStrict>
-__device__ __forceinline__ uint32_t count_bits(const uint64_t (&cd)[kRegBatches], uint32_t nbat,
+__device__ __forceinline__ uint32_t count_bits(const uint64_t (&cd)[kGroupBatches], uint32_t nbat,
                                                uint64_t t)
 {
     uint32_t c = 0;
 #pragma unroll
-    for (int b = 0; b < kRegBatches; ++b)
+    for (int b = 0; b < kGroupBatches; ++b)
         if (static_cast<uint32_t>(b) < nbat)
             c += __popcll(__ballot(kStrict ? cd[b] < t : cd[b] <= t));
     return c;
@@ -425,7 +466,7 @@ __device__ __forceinline__ float round_factor(int i)
     return f[i];
 }
 
-__device__ __forceinline__ bool select_count(const uint64_t (&cd)[kRegBatches], uint32_t nbat,
+__device__ __forceinline__ bool select_count(const uint64_t (&cd)[kGroupBatches], uint32_t nbat,
                                              uint32_t fetch, double hint, uint64_t& E)
 {
     const double h = uniform_f64(hint);
@@ -439,7 +480,7 @@ __device__ __forceinline__ bool select_count(const uint64_t (&cd)[kRegBatches], 
         c[i] = 0;
     }
 #pragma unroll
-    for (int b = 0; b < kRegBatches; ++b) {
+    for (int b = 0; b < kGroupBatches; ++b) {
         if (static_cast<uint32_t>(b) >= nbat) break;
 #pragma unroll
         for (int i = 0; i < kRound; ++i) c[i] += __popcll(__ballot(cd[b] <= tb[i]));
@@ -475,24 +516,24 @@ __device__ __forceinline__ bool select_count(const uint64_t (&cd)[kRegBatches], 
         // Few candidates inside the bracket: each ranks itself among them
         // (strictly smaller ones), and the one at rank fetch - clo - 1 is the
         // fetch-th distance when it is alone there; checked by its count.
-        uint64_t mb[kRegBatches];
-        uint32_t rk[kRegBatches];
+        uint64_t mb[kGroupBatches];
+        uint32_t rk[kGroupBatches];
 #pragma unroll
-        for (int b = 0; b < kRegBatches; ++b) {
+        for (int b = 0; b < kGroupBatches; ++b) {
             rk[b] = 0;
             mb[b] = static_cast<uint32_t>(b) < nbat
                         ? __ballot((ilo < 0 || cd[b] > lob) && cd[b] <= hib)
                         : 0ull;
         }
 #pragma unroll
-        for (int b = 0; b < kRegBatches; ++b) {
+        for (int b = 0; b < kGroupBatches; ++b) {
             uint64_t m = mb[b];
             while (m) {
                 const int l = __builtin_ctzll(m);
                 m &= m - 1;
                 const uint64_t v = lane_u64(cd[b], l);
 #pragma unroll
-                for (int b2 = 0; b2 < kRegBatches; ++b2)
+                for (int b2 = 0; b2 < kGroupBatches; ++b2)
                     if (static_cast<uint32_t>(b2) < nbat) rk[b2] += v < cd[b2] ? 1u : 0u;
             }
         }
@@ -500,14 +541,14 @@ __device__ __forceinline__ bool select_count(const uint64_t (&cd)[kRegBatches], 
         uint64_t pick = kInfD;
         uint32_t npick = 0;
 #pragma unroll
-        for (int b = 0; b < kRegBatches; ++b) {
+        for (int b = 0; b < kGroupBatches; ++b) {
             if (static_cast<uint32_t>(b) >= nbat) break;
             const uint64_t m = mb[b] & __ballot(rk[b] == want);
             npick += static_cast<uint32_t>(__popcll(m));
             if (m && pick == kInfD) pick = lane_u64(cd[b], __builtin_ctzll(m));
         }
         if (npick == 1) {
-                    if (count_bits<false>(cd, nbat, pick) == fetch) {
+            if (count_bits<false>(cd, nbat, pick) == fetch) {
                 E = pick;
                 return true;
             }
@@ -532,7 +573,7 @@ __device__ __forceinline__ bool select_count(const uint64_t (&cd)[kRegBatches], 
             const uint64_t lb = d2_bits(lo), hb = d2_bits(hi);
             uint64_t piv = kInfD;
 #pragma unroll
-            for (int b = 0; b < kRegBatches; ++b) {
+            for (int b = 0; b < kGroupBatches; ++b) {
                 if (static_cast<uint32_t>(b) >= nbat || piv != kInfD) continue;
                 const uint64_t m = __ballot(cd[b] > lb && cd[b] < hb);
                 if (m) piv = lane_u64(cd[b], __builtin_ctzll(m));
@@ -541,7 +582,7 @@ __device__ __forceinline__ bool select_count(const uint64_t (&cd)[kRegBatches], 
             t = bits_d2(piv);
         }
         const uint64_t tbt = d2_bits(t);
-            const uint32_t ct = count_bits<false>(cd, nbat, tbt);
+        const uint32_t ct = count_bits<false>(cd, nbat, tbt);
         if (ct == fetch) {
             E = tbt;
             return true;
@@ -620,7 +661,7 @@ __device__ __forceinline__ void search_single(const KnnArgs& a, const WaveGrid& 
         best = ent_inf();
         for (int cb = 0; cb < ncb; cb += 64) {
             uint32_t lo, len;
-            box_ranges(a, wg, b, cb, lane, lo, len);
+            box_ranges(a, wg, b, cb, lane, static_cast<uint32_t>(a.tune.small_col), lo, len);
             const uint32_t incl = wave_incl_scan_u32(len, lane);
             const uint32_t tot = lane_u32(incl, 63);
             const uint32_t excl = incl - len;
@@ -739,80 +780,862 @@ __device__ __forceinline__ void finish_query(const KnnArgs& a, const WaveGrid& w
     }
 }
 
-template <bool kTiled, int kWaves>
-// Four waves per SIMD: the selection is a chain of ballots and LDS
-// round trips, so more resident waves hide more of its latency (measured
-// faster than three waves even with the register spills four waves cost).
-__global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_knn(KnnArgs a_in)
+// The tile holding sorted row s.
+__device__ __forceinline__ uint32_t tile_of(const uint64_t* __restrict__ starts, uint32_t T,
+                                            uint64_t s)
 {
-    extern __shared__ uint32_t s_lds[];
-    const int lane = __lane_id();
-    // Wave-uniform by construction; said so, so that per-wave tables load
-    // into scalar registers.
-    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
-    const int Q = a_in.q_per_wave;
-    const uint32_t lb = xcd_logical_block(blockIdx.x, gridDim.x);
-    const uint64_t task = static_cast<uint64_t>(lb) * kWaves + w;
-    const KnnArgs& a = a_in;
-    WaveGrid wg;
-    uint64_t q0;
-    int nq;
+    uint32_t lo = 0, hi = T;  // largest t with starts[t] <= s
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (starts[mid] <= s)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+__device__ __forceinline__ void tile_grid(const KnnArgs& a, const TileInfo& ti, WaveGrid& wg)
+{
+    wg.g = ti.g;
+    wg.colstart = a.cv.colstart + ti.colbase;
+    wg.margin = ti.margin;
+    wg.fetch = ti.prog.fetch;
+    wg.k = ti.prog.k;
+    wg.stride = ti.prog.stride;
+}
+
+__device__ __forceinline__ void cloud_grid(const KnnArgs& a, WaveGrid& wg)
+{
+    wg.g = a.cv.g;
+    wg.colstart = a.cv.colstart;
+    wg.margin = a.margin;
+    wg.fetch = a.prog.fetch;
+    wg.k = a.prog.k;
+    wg.stride = a.prog.stride;
+}
+
+// The wave's queries [q0, q0 + nq) and its cloud's or tile's grid and
+// program; false for a task past the last one.
+template <bool kTiled>
+__device__ __forceinline__ bool wave_queries(const KnnArgs& a, uint64_t task, int Q, WaveGrid& wg,
+                                             uint64_t& q0, int& nq)
+{
     if (kTiled) {
-        // The wave's queries and its tile's grid and program.
-        if (task >= a_in.ntasks) return;
+        if (task >= a.ntasks) return false;
         // The task's tile: the last t with task0[t] <= task (tiles with no
         // task share the next tile's prefix).
-        uint32_t tlo = 0, thi = a_in.ntiles;
+        uint32_t tlo = 0, thi = a.ntiles;
         while (thi - tlo > 1) {
             const uint32_t mid = (tlo + thi) >> 1;
-            if (a_in.task0[mid] <= task)
+            if (a.task0[mid] <= task)
                 tlo = mid;
             else
                 thi = mid;
         }
-        const TileInfo& ti = a_in.tiles[tlo];
-        const uint64_t first = static_cast<uint64_t>(task - a_in.task0[tlo]) * Q;
-        wg.g = ti.g;
-        wg.colstart = a_in.cv.colstart + ti.colbase;
-        wg.margin = ti.margin;
-        wg.fetch = ti.prog.fetch;
-        wg.k = ti.prog.k;
-        wg.stride = ti.prog.stride;
+        const TileInfo& ti = a.tiles[tlo];
+        const uint64_t first = (task - a.task0[tlo]) * static_cast<uint64_t>(Q);
+        tile_grid(a, ti, wg);
         q0 = ti.start + first;
         nq = static_cast<int>(ti.n - first < static_cast<uint64_t>(Q) ? ti.n - first : Q);
-    } else {
-        wg.g = a_in.cv.g;
-        wg.colstart = a_in.cv.colstart;
-        wg.margin = a_in.margin;
-        wg.fetch = a_in.prog.fetch;
-        wg.k = a_in.prog.k;
-        wg.stride = a_in.prog.stride;
-        const uint64_t n = a_in.cv.n;
-        q0 = task * Q;
-        if (q0 >= n) return;
-        nq = static_cast<int>(n - q0 < static_cast<uint64_t>(Q) ? n - q0 : Q);
+        return true;
     }
+    cloud_grid(a, wg);
+    q0 = task * static_cast<uint64_t>(Q);
+    if (q0 >= a.cv.n) return false;
+    nq = static_cast<int>(a.cv.n - q0 < static_cast<uint64_t>(Q) ? a.cv.n - q0 : Q);
+    return true;
+}
+
+// ------------------------------------------------- query-per-lane search --
+//
+// A wave takes Q (<= 64) consecutive sorted queries, one per lane.  The
+// queries' bounding box grown by a search radius r is staged once in LDS: the
+// FP64 coordinates and sorted positions of the points inside it,
+// counting-sorted into small cells (x fastest), so that the cells a query can
+// see in one row are one contiguous run.  Every lane then walks its own runs
+// -- the rows (and, in tall boxes, layers) within its own radius rl <= r,
+// chosen from the number of points around it -- computes KD3Index's FP64
+// squared distances and appends (distance, slot) to its own list when below
+// its bound E (at first rl * rl).  A list that fills up is sorted in registers
+// (a compile-time merge-exchange network over 32-bit keys: the distance as
+// FP32 without its low bits, the slot in their place) and cut back to the
+// fetch + 1 + kLaneSlack smallest, and the bound drops to the largest of them.
+//
+// The 32-bit keys only order coarsely; at the end the kept entries' FP64
+// distances are put into (d2, id) order exactly.  A row is final when its
+// fetch-th distance is below its radius squared and its (fetch + 1)-th below
+// every entry cut away.  The radius is at most the ring_max cells that bound
+// the growing search, so a row found here is one that search would certify.
+// A group whose box holds too many points is halved along its longest axis.
+// A few lanes not final go to k_knn_rest; more of them are tried again with
+// a larger radius first.
+//
+// Bound by vector instructions (staging, walks and the sorting network) at two
+// waves per SIMD.  Against the wave-per-query search (k_knn_group) for every
+// row, search time: 4M points k 16 8.4 -> 5.4 ms, 777k k 8 stride 3 3.6 ->
+// 2.2, 250k k 10 1.67 -> 0.64; 10M points of terrain and flat roofs, k 32,
+// 34 -> 32.
+constexpr int kLaneSlack = 2;   // entries beyond fetch + 1 put in exact order
+// First radius over the one the density's estimate gives, and the points a
+// lane's radius should hold over fetch + 1 (measured best of 1.2 to 1.7 and 1.5
+// to 2.1: smaller ones fail lanes, larger ones fill boxes and lists).
+constexpr float kRadiusFactor = 1.35f;
+constexpr float kListFactor = 1.8f;
+constexpr int kLaneTries = 3;   // radii tried per query
+constexpr int kLaneFew = 6;     // lanes not worth another round of their own
+constexpr uint32_t kStageMax = 512;    // points staged per round
+constexpr int kStageSlots = 16;        // points of the box's columns per lane and round
+constexpr uint32_t kStageRaw = kStageSlots * 64;
+constexpr uint32_t kStageCells = 512;
+constexpr int kStageCols = 5;          // columns of a box per lane
+constexpr int kListRow = 65;    // LDS words between list positions of the ordered lists
+constexpr uint32_t kSlotMask = 0x3FFu;  // slot in a key's low bits (kStageMax <= 1024)
+
+template <int P, int Q, int R, int D, int N>
+__device__ __forceinline__ void sort_step(uint32_t (&k)[N])
+{
+#pragma unroll
+    for (int i = 0; i < N - D; ++i)
+        if ((i & P) == R) {
+            const uint32_t a = min(k[i], k[i + D]), b = max(k[i], k[i + D]);
+            k[i] = a;
+            k[i + D] = b;
+        }
+    if constexpr (Q != P) sort_step<P, Q / 2, P, Q - P, N>(k);
+}
+
+template <int P, int T, int N> __device__ __forceinline__ void sort_phase(uint32_t (&k)[N])
+{
+    if constexpr (P > 0) {
+        sort_step<P, T, 0, P, N>(k);
+        sort_phase<P / 2, T, N>(k);
+    }
+}
+
+constexpr int half_pow2(int n)  // largest power of two below n
+{
+    int t = 1;
+    while (2 * t < n) t *= 2;
+    return t;
+}
+
+// Ascending sort of N registers (Knuth's merge exchange, algorithm 5.2.2M).
+template <int N> __device__ __forceinline__ void sort_net(uint32_t (&k)[N])
+{
+    constexpr int T = half_pow2(N);
+    sort_phase<T, T, N>(k);
+}
+
+// Reductions and scans over the whole wave by data-parallel moves within the
+// register file (rows of 16 lanes, then the rows' last lanes); every lane
+// must be active.
+template <int kCtrl, int kRows> __device__ __forceinline__ uint32_t dpp_u32(uint32_t old, uint32_t v)
+{
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+        static_cast<int>(old), static_cast<int>(v), kCtrl, kRows, 0xF, false));
+}
+
+__device__ __forceinline__ float wave_min_f32(float v)
+{
+    auto step = [&](uint32_t o) { v = fminf(v, __uint_as_float(o)); };
+    step(dpp_u32<0x111, 0xF>(__float_as_uint(v), __float_as_uint(v)));
+    step(dpp_u32<0x112, 0xF>(__float_as_uint(v), __float_as_uint(v)));
+    step(dpp_u32<0x114, 0xF>(__float_as_uint(v), __float_as_uint(v)));
+    step(dpp_u32<0x118, 0xF>(__float_as_uint(v), __float_as_uint(v)));
+    step(dpp_u32<0x142, 0xA>(__float_as_uint(v), __float_as_uint(v)));
+    step(dpp_u32<0x143, 0xC>(__float_as_uint(v), __float_as_uint(v)));
+    return __uint_as_float(lane_u32(__float_as_uint(v), 63));
+}
+
+// Extent of v over the active lanes of the first and second half of the
+// wave's queries: halves of the wave, or (two lanes per query) of its first
+// half.
+template <int LPQ> __device__ __forceinline__ float2 half_extents(bool act, float v)
+{
+    float lo = act ? v : INFINITY, hi = act ? -v : INFINITY;
+    auto step = [&](float& m, uint32_t o) { m = fminf(m, __uint_as_float(o)); };
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        float& m = i ? hi : lo;
+        step(m, dpp_u32<0x111, 0xF>(__float_as_uint(m), __float_as_uint(m)));
+        step(m, dpp_u32<0x112, 0xF>(__float_as_uint(m), __float_as_uint(m)));
+        step(m, dpp_u32<0x114, 0xF>(__float_as_uint(m), __float_as_uint(m)));
+        step(m, dpp_u32<0x118, 0xF>(__float_as_uint(m), __float_as_uint(m)));
+        if (LPQ == 1) step(m, dpp_u32<0x142, 0xA>(__float_as_uint(m), __float_as_uint(m)));
+    }
+    const float e = -hi - lo;
+    return make_float2(__uint_as_float(lane_u32(__float_as_uint(e), LPQ == 1 ? 31 : 15)),
+                       __uint_as_float(lane_u32(__float_as_uint(e), LPQ == 1 ? 63 : 31)));
+}
+
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v)
+{
+    v += dpp_u32<0x111, 0xF>(0u, v);
+    v += dpp_u32<0x112, 0xF>(0u, v);
+    v += dpp_u32<0x114, 0xF>(0u, v);
+    v += dpp_u32<0x118, 0xF>(0u, v);
+    v += dpp_u32<0x142, 0xA>(0u, v);
+    v += dpp_u32<0x143, 0xC>(0u, v);
+    return v;
+}
+
+// The lane's list (LDS, one column per lane), sorted; its entries after cnt
+// read as the largest key.
+template <int CAP>
+__device__ __forceinline__ void load_sorted(const uint32_t* my, uint32_t cnt, uint32_t (&k)[CAP])
+{
+#pragma unroll
+    for (int i = 0; i < CAP; ++i) {
+        const uint32_t v = my[i * 64];
+        k[i] = static_cast<uint32_t>(i) < cnt ? v : kInfU;
+    }
+    sort_net<CAP>(k);
+}
+
+template <int CAP> struct StageShared {
+    double x[kStageMax], y[kStageMax], z[kStageMax];
+    uint32_t j[kStageMax];
+    uint32_t cell[kStageCells + 2];   // counts, then first slots; last: points left out
+    union {
+        uint32_t list[CAP * 64];      // one list column per lane
+        uint32_t pos[kStageRaw];      // while staging: sorted positions of the box's columns
+    };
+};
+
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// FP64 covariance of the k neighbors pos(0..k-1) (indexes into x, y, z;
+// two-pass mean) into sorted row s's record, with its search flags.  Coordinates are taken
+// relative to the query point (exact differences at any offset), so the mean
+// carries no rounding of the cloud's absolute position: at UTM scale that
+// rounding (~1e-9 m) would add a rank-one term to the covariance of flat and
+// collinear neighborhoods.
+template <class Pos>
+__device__ __forceinline__ void write_cov_record(const KnnArgs& a, uint64_t s, int k, double ox,
+                                                 double oy, double oz, uint8_t flags,
+                                                 const double* x, const double* y,
+                                                 const double* z, Pos pos)
+{
+    double mx = 0.0, my = 0.0, mz = 0.0;
+#pragma unroll 4
+    for (int l = 0; l < k; ++l) {
+        const uint32_t j = pos(l);
+        mx += x[j] - ox;
+        my += y[j] - oy;
+        mz += z[j] - oz;
+    }
+    mx /= static_cast<double>(k);
+    my /= static_cast<double>(k);
+    mz /= static_cast<double>(k);
+    double c[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll 4
+    for (int l = 0; l < k; ++l) {
+        const uint32_t j = pos(l);
+        const double dx = (x[j] - ox) - mx, dy = (y[j] - oy) - my,
+                     dz = (z[j] - oz) - mz;
+        c[0] += dx * dx;
+        c[1] += dx * dy;
+        c[2] += dx * dz;
+        c[3] += dy * dy;
+        c[4] += dy * dz;
+        c[5] += dz * dz;
+    }
+    const double den = static_cast<double>(k - 1);
+    double* rec = a.out.cov + kCovRecord * s;
+    for (int i = 0; i < 6; ++i) rec[i] = c[i] / den;
+    reinterpret_cast<uint64_t*>(rec)[6] = flags;
+}
+
+// The final rows of a wave: lists of slots (LDS, 65 words between positions,
+// so that lanes read a position and rows read a list without bank conflicts)
+// to covariance records or to the output lists.
+__device__ __forceinline__ void store_rows(const KnnArgs& a, const WaveGrid& wg, uint64_t s,
+                                           int lane, bool done, bool tie, double qx, double qy,
+                                           double qz, const double* x, const double* y,
+                                           const double* z, const uint32_t* sj,
+                                           const uint32_t* list)
+{
+    const uint64_t dm = __ballot(done);
+    if (!dm) return;
+    const uint8_t flags = tie ? ST_TIE : 0;
+    const int stride = wg.stride;
+    if (a.mode == 0) {
+        if (done)
+            write_cov_record(a, s, wg.k, qx, qy, qz, flags, x, y, z,
+                             [&](int l) { return list[l * stride * kListRow + lane]; });
+    } else {
+        const uint32_t qid = done ? a.cv.perm[s] : 0u;
+        if (done) a.out.status[0][qid] = flags;
+        // One row after another, its k entries side by side.
+        for (uint64_t m = dm; m; m &= m - 1) {
+            const int r = __builtin_ctzll(m);
+            const uint64_t row = lane_u32(qid, r);
+            if (lane < wg.k) {
+                const uint32_t j = sj[list[lane * stride * kListRow + r]];
+                a.out.ids[row * static_cast<uint64_t>(wg.k) + lane] =
+                    a.mode == 2 ? j : a.cv.perm[j];
+            }
+        }
+    }
+    const uint64_t tm = __ballot(done && tie);
+    if (tm) {
+        uint32_t at = 0;
+        if (lane == 0) {
+            const uint32_t c = static_cast<uint32_t>(__popcll(tm));
+            at = atomicAdd(a.out.nflagged, c);
+            atomicAdd(a.out.nflagged + 1, c);
+        }
+        at = lane_u32(at, 0) + lanes_below64(tm);
+        if (done && tie) a.out.flagged[at] = static_cast<uint32_t>(s);
+    }
+}
+
+// The search of one group of queries [q0, q0 + nq); LPQ lanes per query (the
+// second lane of a pair takes every other candidate, and the pair's two
+// lists are merged before the exact order).  With kBail a group whose first
+// box holds too many points is left whole: returns true, nothing written.
+template <int CAP, int TM, int LPQ, bool kBail>
+__device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& wg, uint64_t q0,
+                                             int nq, StageShared<CAP>& S)
+{
+    const int lane = __lane_id();
+    const int ql = lane & (64 / LPQ - 1);  // the lane's query
+    const int part = LPQ == 1 ? 0 : lane >> 5;
+    const CloudView& cv = a.cv;
+    const GridParams& g = wg.g;
+    const uint32_t fetch = static_cast<uint32_t>(wg.fetch);
+    const uint32_t keep = fetch + 1 + kLaneSlack;  // <= TM
+    const bool valid = ql < nq;
+    const uint64_t s = valid ? cv.qord[q0 + ql] : q0;
+    const double qx = valid ? cv.sx[s] : 0.0;
+    const double qy = valid ? cv.sy[s] : 0.0;
+    const double qz = valid ? cv.sz[s] : 0.0;
+    const uint32_t key0 = cv.keys[uniform_u32(cv.qord[q0])];
+    uint32_t* my = S.list + lane;
+    // The growing search's box reaches ring_max whole cells from a query's
+    // own cell on every side.
+    const float r_cap = static_cast<float>(
+        (static_cast<double>(a.tune.ring_max) * fmin(g.c, g.cz) - 4.0 * wg.margin) * (1.0 - 1e-6));
+    bool pending = valid && isfinite(qx) && isfinite(qy) && isfinite(qz) && r_cap > 0.0f;
+    bool defer = valid && !pending;
+    uint32_t tries = 0;
+    float r_need = 0.0f;  // the smallest radius worth trying for this lane
+    // The first radius, from two densities around the wave: of a surface (the
+    // first query's 8 x 8 columns), and of a volume (the denser half of the
+    // wave's queries in its bounding box).
+    float r_first = r_cap;
+    {
+        const uint32_t t = (key0 >> g.bz) >> 6;
+        const uint32_t n8 = wg.colstart[64 * t + 64] - wg.colstart[64 * t];
+        const uint32_t tx = t % g.tiles_x, ty = t / g.tiles_x;
+        const float cf = static_cast<float>(g.c);
+        const float area = static_cast<float>(min(8u, g.gx - 8 * tx)) *
+                           static_cast<float>(min(8u, g.gy - 8 * ty)) * cf * cf;
+        const float per = static_cast<float>(fetch + 1);
+        const float r2 = sqrtf(per * area * 0.31830989f / static_cast<float>(max(n8, 1u)));
+        const double bx = lane_value(qx, 0), by = lane_value(qy, 0), bz = lane_value(qz, 0);
+        const float dx = static_cast<float>(qx - bx), dy = static_cast<float>(qy - by),
+                    dz = static_cast<float>(qz - bz);
+        const float2 ex = half_extents<LPQ>(pending, dx), ey = half_extents<LPQ>(pending, dy),
+                     ez = half_extents<LPQ>(pending, dz);
+        const uint64_t vm = __ballot(pending);
+        const int half = __popcll(vm & (LPQ == 1 ? 0xFFFFFFFFull : 0xFFFFull));
+        const int rest = __popcll((LPQ == 1 ? vm >> 32 : vm >> 16) & (LPQ == 1 ? 0xFFFFFFFFull : 0xFFFFull));
+        const float va = half ? ex.x * ey.x * ez.x / static_cast<float>(half) : INFINITY;
+        const float vb = rest ? ex.y * ey.y * ez.y / static_cast<float>(rest) : INFINITY;
+        const float v = fminf(va, vb);
+        const float r3 = v < INFINITY ? cbrtf(per * v * 0.23873241f) : 0.0f;
+        r_first = fminf(kRadiusFactor * fmaxf(r2, r3), r_cap);
+    }
+    uint64_t cnt_pass = 0, cnt_cand = 0, cnt_sort = 0;
+    for (int round = 0; round < (kBail ? 2 : 3); ++round) {
+        // The round's group: the pending lanes with as many tries behind them
+        // as the first pending one.
+        const uint64_t pm = __ballot(pending);
+        if (!pm) break;
+        const int first = __builtin_ctzll(pm);
+        const double bx = lane_value(qx, first), by = lane_value(qy, first),
+                     bz = lane_value(qz, first);
+        const float rx = static_cast<float>(qx - bx), ry = static_cast<float>(qy - by),
+                    rz = static_cast<float>(qz - bz);
+        const uint32_t first_tries = lane_u32(tries, first);
+        bool act = pending && tries == first_tries;
+        float r = r_first;
+        double X0 = 0, X1 = 0, Y0 = 0, Y1 = 0, Z0 = 0, Z1 = 0;
+        float hx = 0, hy = 0, hz = 0;  // 1 / cell edges of the staged box
+        int nx = 1, ny = 1, nz = 1;
+        bool got = false;
+        int refine = 0;
+        for (int step = 0; step < 16; ++step) {
+            const float lx = wave_min_f32(act ? rx : INFINITY), ux = -wave_min_f32(act ? -rx : INFINITY);
+            const float ly = wave_min_f32(act ? ry : INFINITY), uy = -wave_min_f32(act ? -ry : INFINITY);
+            const float lz = wave_min_f32(act ? rz : INFINITY), uz = -wave_min_f32(act ? -rz : INFINITY);
+            const float r_need_max = fminf(-wave_min_f32(act ? -r_need : 0.0f), r_cap);
+            r = fmaxf(r, r_need_max);
+            // Faces at least r from every active query: the offsets' FP32
+            // rounding and the FP64 rounding of the faces taken off.
+            const float W = fmaxf(fmaxf(fmaxf(-lx, ux), fmaxf(-ly, uy)), fmaxf(-lz, uz)) + r;
+            const double pad = static_cast<double>(r) + 3e-7 * static_cast<double>(W) + wg.margin;
+            X0 = bx + static_cast<double>(lx) - pad;
+            X1 = bx + static_cast<double>(ux) + pad;
+            Y0 = by + static_cast<double>(ly) - pad;
+            Y1 = by + static_cast<double>(uy) + pad;
+            Z0 = bz + static_cast<double>(lz) - pad;
+            Z1 = bz + static_cast<double>(uz) + pad;
+            // Grid cells by the points' own rule, so that a point inside the
+            // faces is inside the cells.
+            const Box b{uniform_i32(static_cast<int>(cell_coord(X0, g.ox, g.inv_c, g.gx))),
+                        uniform_i32(static_cast<int>(cell_coord(X1, g.ox, g.inv_c, g.gx))),
+                        uniform_i32(static_cast<int>(cell_coord(Y0, g.oy, g.inv_c, g.gy))),
+                        uniform_i32(static_cast<int>(cell_coord(Y1, g.oy, g.inv_c, g.gy))),
+                        uniform_i32(static_cast<int>(cell_coord(Z0, g.oz, g.inv_cz, g.gz))),
+                        uniform_i32(static_cast<int>(cell_coord(Z1, g.oz, g.inv_cz, g.gz)))};
+            const uint64_t ncb = static_cast<uint64_t>(b.x1 - b.x0 + 1) *
+                                 static_cast<uint64_t>(b.y1 - b.y0 + 1);
+            bool over = ncb > kStageCols * 64u;
+            if (!over) {
+                uint32_t lo[kStageCols], len[kStageCols], part = 0;
+                box_columns(a, wg, b, static_cast<int>(ncb), lane, lo, len);
+#pragma unroll
+                for (int i = 0; i < kStageCols; ++i) part += min(len[i], 1u << 20);
+                const uint32_t incl = wave_scan_u32(part);
+                const uint32_t N = lane_u32(incl, 63);
+                // Where the box turns out denser than the first estimates, the
+                // radius its own density asks for.
+                if (refine < 2 && r > r_need_max) {
+                    const float ex = static_cast<float>(b.x1 - b.x0 + 1) * static_cast<float>(g.c);
+                    const float ey = static_cast<float>(b.y1 - b.y0 + 1) * static_cast<float>(g.c);
+                    const float ez = static_cast<float>(b.z1 - b.z0 + 1) * static_cast<float>(g.cz);
+                    const float per = static_cast<float>(fetch + 1) / static_cast<float>(max(N, 1u));
+                    const float r2 = sqrtf(per * ex * ey * 0.31830989f);
+                    const float r3 = cbrtf(per * ex * ey * ez * 0.23873241f);
+                    const float rn = fmaxf(kRadiusFactor * fmaxf(r2, r3), r_need_max);
+                    ++refine;
+                    if (rn < 0.85f * r) {
+                        r = fmaxf(rn, 0.5f * r);
+                        continue;
+                    }
+                }
+                over = N > kStageRaw || N == 0;
+                if (!over) {
+                    // Cells: a third of the radius along x (runs are cut
+                    // there), half of it along y, the radius along z when the
+                    // box is tall.
+                    const float Lx = static_cast<float>(X1 - X0), Ly = static_cast<float>(Y1 - Y0),
+                                Lz = static_cast<float>(Z1 - Z0);
+                    float cx = r * 0.34f, cy = r * 0.5f, cz = r;
+                    for (;;) {
+                        nx = uniform_i32(static_cast<int>(fminf(Lx / cx, 1000.0f)) + 1);
+                        ny = uniform_i32(static_cast<int>(fminf(Ly / cy, 1000.0f)) + 1);
+                        nz = uniform_i32(Lz > 4.0f * r ? static_cast<int>(fminf(Lz / cz, 1000.0f)) + 1 : 1);
+                        if (static_cast<uint32_t>(nx * ny * nz) <= kStageCells) break;
+                        cx *= 1.3f;
+                        cy *= 1.3f;
+                        cz *= 1.3f;
+                    }
+                    hx = 1.0f / cx;
+                    hy = 1.0f / cy;
+                    hz = nz > 1 ? 1.0f / cz : 0.0f;
+                    // The columns' points, one per lane and slot.
+                    uint32_t at = incl - part;
+#pragma unroll
+                    for (int i = 0; i < kStageCols; ++i)
+                        for (uint32_t c = 0; c < len[i]; ++c) S.pos[at++] = lo[i] + c;
+#pragma unroll
+                    for (uint32_t c = 0; c < kStageCells; c += 64) S.cell[c + lane] = 0;
+                    wave_lds_order();
+                    // Four points per lane at a time; the coordinates are read
+                    // again (from cache) when the slots are known, so that
+                    // they do not hold registers in between.
+                    uint32_t pc[kStageSlots];  // cell << 16 | rank in it, or ~0
+#pragma unroll
+                    for (int i0 = 0; i0 < kStageSlots; i0 += 4) {
+                        if (i0 * 64u >= N) {  // wave-uniform
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) pc[i0 + i] = ~0u;
+                            continue;
+                        }
+                        double px[4], py[4], pz[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const uint32_t t = (i0 + i) * 64u + lane;
+                            const uint32_t j = S.pos[t < N ? t : 0u];
+                            px[i] = cv.sx[j];
+                            py[i] = cv.sy[j];
+                            pz[i] = cv.sz[j];
+                        }
+                        uint32_t cell[4], rank[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const uint32_t t = (i0 + i) * 64u + lane;
+                            const int ix = min(static_cast<int>(static_cast<float>(px[i] - X0) * hx), nx - 1);
+                            const int iy = min(static_cast<int>(static_cast<float>(py[i] - Y0) * hy), ny - 1);
+                            const int iz = min(static_cast<int>(static_cast<float>(pz[i] - Z0) * hz), nz - 1);
+                            const bool in = static_cast<int>(t < N) & static_cast<int>(px[i] >= X0) &
+                                            static_cast<int>(px[i] <= X1) & static_cast<int>(py[i] >= Y0) &
+                                            static_cast<int>(py[i] <= Y1) & static_cast<int>(pz[i] >= Z0) &
+                                            static_cast<int>(pz[i] <= Z1);
+                            // (points outside count in a cell of their own)
+                            cell[i] = in ? static_cast<uint32_t>((iz * ny + iy) * nx + ix) : kStageCells + 1u;
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) rank[i] = atomicAdd(&S.cell[cell[i]], 1u);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            pc[i0 + i] = cell[i] <= kStageCells ? (cell[i] << 16) | rank[i] : ~0u;
+                    }
+                    wave_lds_order();
+                    // First slots of the cells (eight cells per lane).
+                    constexpr int kPer = kStageCells / 64;
+                    uint32_t v[kPer], sum = 0;
+#pragma unroll
+                    for (int i = 0; i < kPer; ++i) {
+                        v[i] = S.cell[lane * kPer + i];
+                        sum += v[i];
+                    }
+                    uint32_t ex = wave_scan_u32(sum);
+                    const uint32_t M = lane_u32(ex, 63);
+                    ex -= sum;
+#pragma unroll
+                    for (int i = 0; i < kPer; ++i) {
+                        S.cell[lane * kPer + i] = ex;
+                        ex += v[i];
+                    }
+                    if (lane == 0) S.cell[kStageCells] = M;
+                    wave_lds_order();
+                    over = M > kStageMax;
+                    if (!over) {
+#pragma unroll
+                        for (int i0 = 0; i0 < kStageSlots; i0 += 4) {
+                            if (i0 * 64u >= N) break;
+                            double px[4], py[4], pz[4];
+                            uint32_t j[4], at[4];
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const uint32_t t = (i0 + i) * 64u + lane;
+                                j[i] = S.pos[t < N ? t : 0u];
+                                px[i] = cv.sx[j[i]];
+                                py[i] = cv.sy[j[i]];
+                                pz[i] = cv.sz[j[i]];
+                                const uint32_t c = pc[i0 + i];
+                                at[i] = c != ~0u ? S.cell[c >> 16] + (c & 0xFFFFu) : ~0u;
+                            }
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                if (at[i] != ~0u) {
+                                    S.x[at[i]] = px[i];
+                                    S.y[at[i]] = py[i];
+                                    S.z[at[i]] = pz[i];
+                                    S.j[at[i]] = j[i];
+                                }
+                            }
+                        }
+                        wave_lds_order();
+                    }
+                }
+            }
+            if (!over) {
+                got = true;
+                break;
+            }
+            if (kBail && round == 0) return true;
+            // Too many: the half of the group that holds its first query.
+            const float dx = ux - lx, dy = uy - ly, dz = uz - lz;
+            const float big = fmaxf(dx, fmaxf(dy, dz));
+            if (!(big > 0.0f)) break;  // all at one place
+            const float v = dx == big ? rx : (dy == big ? ry : rz);
+            const float mid = 0.5f * (dx == big ? lx + ux : (dy == big ? ly + uy : lz + uz));
+            // (the first query is the base: its offset is 0)
+            act = act && (v <= mid) == (0.0f <= mid);
+        }
+        if (!got) {
+            defer |= act;
+            pending = pending && !act;
+            continue;
+        }
+        // The lane's cells at radius rl: rows and layers [*0, *1].
+        float rl = r;
+        int cx0 = 0, cx1 = 0, cy0 = 0, cy1 = -1, cz0 = 0, cz1 = 0;
+        const float fx = static_cast<float>(qx - X0), fy = static_cast<float>(qy - Y0),
+                    fz = static_cast<float>(qz - Z0);
+        auto cells = [&](float rr) {
+            // A hair wider than rr, so that rounding loses no point.
+            const float e = rr * 1.0001f + 1e-6f * (fabsf(fx) + fabsf(fy) + fabsf(fz)) +
+                            static_cast<float>(wg.margin);
+            cx0 = min(static_cast<int>(fmaxf(fx - e, 0.0f) * hx), nx - 1);
+            cx1 = min(static_cast<int>((fx + e) * hx), nx - 1);
+            cy0 = static_cast<int>(fmaxf(fy - e, 0.0f) * hy);
+            cy1 = act ? min(static_cast<int>((fy + e) * hy), ny - 1) : cy0 - 1;
+            cz0 = min(static_cast<int>(fmaxf(fz - e, 0.0f) * hz), nz - 1);
+            cz1 = act ? min(static_cast<int>((fz + e) * hz), nz - 1) : cz0 - 1;
+        };
+        cells(r);
+        // Where the box is denser around this query than its radius asks for,
+        // a smaller one.
+        {
+            uint32_t seen = 0;
+            for (int z = cz0; z <= cz1; ++z)
+                for (int y = cy0; y <= cy1; ++y) {
+                    const int row = (z * ny + y) * nx;
+                    seen += S.cell[row + cx1 + 1] - S.cell[row + cx0];
+                }
+            // At least a quarter of those seen are inside the radius, and
+            // their number falls at most with its cube.
+            const float in = 0.25f * static_cast<float>(seen);
+            const float want = kListFactor * static_cast<float>(fetch + 1);
+            if (in > want) {
+                rl = fminf(fmaxf(r * cbrtf(want / in), r_need), r);
+                cells(rl);
+            }
+        }
+        cnt_pass += static_cast<uint64_t>(__popcll(__ballot(act)));
+        // The walk.
+        const double E0 = static_cast<double>(rl) * static_cast<double>(rl);
+        double E = act ? E0 : -1.0;
+        uint32_t cnt = 0, seen = 0;
+        bool cut = false;   // entries below E0 may have been left out
+        for (int dz = 0; __ballot(cz0 + dz <= cz1); ++dz) {
+            for (int dy = 0; __ballot(cy0 + dy <= cy1); ++dy) {
+                uint32_t p = 0, e = 0;
+                if (cy0 + dy <= cy1 && cz0 + dz <= cz1) {
+                    const int row = ((cz0 + dz) * ny + cy0 + dy) * nx;
+                    p = S.cell[row + cx0] + part;
+                    e = S.cell[row + cx1 + 1];
+                    seen += e - p;
+                }
+                while (__ballot(p < e)) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t t = p < e ? p : 0u;
+                        const uint64_t db = dist_bits(qx, qy, qz, S.x[t], S.y[t], S.z[t]);
+                        const double d2 = bits_d2(db);
+                        my[cnt * 64] = (__float_as_uint(static_cast<float>(d2)) & ~kSlotMask) | t;
+                        cnt += (p < e && d2 < E) ? 1u : 0u;
+                        p += LPQ;
+                    }
+                    if (__ballot(cnt > CAP - 4)) {
+                        uint32_t k[CAP];
+                        load_sorted<CAP>(my, cnt, k);
+                        cnt_sort += 1;
+#pragma unroll
+                        for (int i = 0; i < TM; ++i) my[i * 64] = k[i];
+                        if (cnt >= keep) {
+                            // (the key's bucket ends below this)
+                            E = fmin(E, static_cast<double>(__uint_as_float(
+                                            (my[(keep - 1) * 64] | kSlotMask) + 1u)));
+                            cnt = keep;
+                            cut = true;
+                        }
+                    }
+                }
+            }
+        }
+        cnt_cand += seen;
+        uint32_t idx[TM];
+        uint64_t d[TM];
+        {
+            uint32_t k[CAP];
+            load_sorted<CAP>(my, cnt, k);
+            cnt_sort += 1;
+            if (LPQ == 2) {
+                // The TM smallest of the pair's two lists.
+                uint32_t m[TM];
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    m[i] = min(k[i], static_cast<uint32_t>(__shfl_xor(static_cast<int>(k[TM - 1 - i]), 32)));
+                sort_net<TM>(m);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) k[i] = m[i];
+                cnt += static_cast<uint32_t>(__shfl_xor(static_cast<int>(cnt), 32));
+                const int other_cut = __shfl_xor(cut ? 1 : 0, 32);
+                cut = cut || other_cut != 0;
+            }
+            const uint32_t lim = min(cnt, keep);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                my[i * 64] = k[i];
+                const bool has = static_cast<uint32_t>(i) < lim;
+                const uint32_t t = has ? k[i] & kSlotMask : 0u;
+                const uint64_t v = dist_bits(qx, qy, qz, S.x[t], S.y[t], S.z[t]);
+                idx[i] = has ? t : kInfU;
+                d[i] = has ? v : kInfD;
+                if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // The largest coarse distance put in exact order: no entry cut away
+        // has a smaller one (the float rounds a double by 6e-8).
+        cut = cut || cnt >= keep;
+        const double last = static_cast<double>(__uint_as_float(my[(keep - 1) * 64] & ~kSlotMask)) *
+                            (1.0 - 1.2e-7);
+        // Exact (d2, id) order: neighbors out of order change places
+        // until none is (the coarse order is right but for near-equal
+        // distances).
+        for (int pass = 0; pass < TM; ++pass) {
+            bool any = false;
+#pragma unroll
+            for (int i = 1; i < TM; ++i) {
+                bool sw = d[i] < d[i - 1];
+                const bool eq = d[i] == d[i - 1] && d[i] != kInfD;
+                if (__ballot(eq)) {
+                    if (eq) sw = cv.perm[S.j[idx[i]]] < cv.perm[S.j[idx[i - 1]]];
+                }
+                const uint64_t u = sw ? d[i] : d[i - 1], v = sw ? d[i - 1] : d[i];
+                const uint32_t iu = sw ? idx[i] : idx[i - 1], iv = sw ? idx[i - 1] : idx[i];
+                d[i - 1] = u;
+                d[i] = v;
+                idx[i - 1] = iu;
+                idx[i] = iv;
+                any |= sw;
+            }
+            if (!__ballot(any)) break;
+        }
+        // In (d2, id) order; the list holds slots now.
+        uint32_t* list = S.list;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < TM; ++i) list[i * kListRow + lane] = idx[i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        // The fetch-th and (fetch + 1)-th distances.
+        auto dist_at = [&](uint32_t i) {
+            const uint32_t t = list[i * kListRow + lane];
+            return t == kInfU ? kInfD : dist_bits(qx, qy, qz, S.x[t], S.y[t], S.z[t]);
+        };
+        const uint64_t dk = dist_at(fetch - 1), dn = dist_at(fetch);
+        bool tie = dk == dn && dk != kInfD;
+        if (wg.stride > 1 || a.mode == 2) {  // equal neighbors anywhere in the list
+            tie = false;
+#pragma unroll
+            for (int i = 1; i < TM; ++i)
+                tie |= static_cast<uint32_t>(i) <= fetch && d[i] == d[i - 1] && d[i] != kInfD;
+        }
+        // (points outside the staged box are farther than rl but for the
+        // rounding of one distance)
+        const bool in_ball = act && cnt >= fetch && bits_d2(dk) < E0 * (1.0 - 1e-12);
+        const bool done = in_ball && (!cut || (dn != kInfD && bits_d2(dn) < last));
+        store_rows(a, wg, s, lane, done && part == 0, tie, qx, qy, qz, S.x, S.y, S.z, S.j, list);
+        // What is left: a larger radius, or the growing search.
+        const bool again = act && !done;
+        const bool few = __popcll(__ballot(again && part == 0)) <= kLaneFew;
+        if (again) {
+            ++tries;
+            const float f = sqrtf(1.5f * static_cast<float>(fetch) /
+                                  static_cast<float>(max(cnt, 1u)));
+            const bool give_up = few || in_ball || tries >= kLaneTries || rl >= r_cap;
+            r_need = rl * fminf(fmaxf(f, 1.3f), 2.0f);
+            defer |= give_up;
+            pending = !give_up;
+        } else if (done) {
+            pending = false;
+        }
+        wave_lds_order();  // the next round stages over this one's box
+    }
+    defer |= pending;  // not reached: every round settles or counts a try of a lane
+    defer = defer && part == 0;
+    const uint64_t dm = __ballot(defer);
+    if (dm) {
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(a.out.nflagged + 3, static_cast<uint32_t>(__popcll(dm)));
+        at = lane_u32(at, 0) + lanes_below64(dm);
+        if (defer) a.out.deferred[at] = static_cast<uint32_t>(s);
+    }
+    if (a.out.counters) {
+        atomicAdd(a.out.counters + 1, static_cast<unsigned long long>(cnt_cand));
+        if (lane == 0) {
+            atomicAdd(a.out.counters + 0, static_cast<unsigned long long>(cnt_pass));
+            atomicAdd(a.out.counters + 2, static_cast<unsigned long long>(cnt_sort));
+            atomicAdd(a.out.counters + 3, static_cast<unsigned long long>(nq));
+        }
+    }
+    return false;
+}
+
+// One group per wave; groups too heavy for one box are listed in out.heavy.
+template <int CAP, int TM, int WPE, bool kTiled>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+void k_knn_lane(KnnArgs a)
+{
+    __shared__ StageShared<CAP> S;
+    const uint32_t task = xcd_logical_block(blockIdx.x, gridDim.x);
+    WaveGrid wg;
+    uint64_t q0;
+    int nq;
+    if (!wave_queries<kTiled>(a, task, a.q_per_wave, wg, q0, nq)) return;
+    if (kTiled && (wg.fetch > a.fetch_hi || wg.fetch < a.fetch_lo)) return;
+    if (search_group<CAP, TM, 1, true>(a, wg, q0, nq, S) && __lane_id() == 0)
+        a.out.heavy[atomicAdd(a.out.nflagged + 4, 1u)] = task;
+}
+
+// The heavy groups, half a group at a time with two lanes per query: half
+// the queries need a smaller box, and each walks it in half the steps.  The
+// waves draw halves until none is left (their number is read on the device).
+template <int CAP, int TM, int WPE, bool kTiled>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+void k_knn_pair(KnnArgs a)
+{
+    __shared__ StageShared<CAP> S;
+    const uint32_t halves = 2u * a.out.nflagged[4];
+    for (;;) {
+        uint32_t h = 0;
+        if (__lane_id() == 0) h = atomicAdd(a.out.nflagged + 7, 1u);
+        h = lane_u32(h, 0);
+        if (h >= halves) return;
+        WaveGrid wg;
+        uint64_t q0;
+        int nq;
+        if (!wave_queries<kTiled>(a, a.out.heavy[h >> 1], a.q_per_wave, wg, q0, nq)) continue;
+        const int first = 32 * static_cast<int>(h & 1u);
+        if (nq <= first) continue;
+        search_group<CAP, TM, 2, false>(a, wg, q0 + first, min(nq - first, 32), S);
+    }
+}
+
+// ------------------------------------------------- wave-per-query search --
+//
+// Neighborhoods too large for the query-per-lane search (more than
+// kLaneMaxFetch entries; its lists and registers grow with them): the
+// wave's queries form groups that share a 2 x 2 block of columns and a short
+// z range, and one candidate box of up to 256 points held in registers; each
+// query's FP64 distances are selected by ballots across the wave.  Rows not
+// certified by that box go to k_knn_rest.
+template <bool kTiled>
+// Four waves per SIMD: the selection is a chain of ballots and LDS round
+// trips, so more resident waves hide more of its latency.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_knn_group(KnnArgs a)
+{
+    extern __shared__ uint32_t s_lds[];
+    const int lane = __lane_id();
+    const int Q = a.q_per_wave;
+    WaveGrid wg;
+    uint64_t q0;
+    int nq;
+    if (!wave_queries<kTiled>(a, xcd_logical_block(blockIdx.x, gridDim.x), Q, wg, q0, nq)) return;
+    if (kTiled && (wg.fetch > a.fetch_hi || wg.fetch < a.fetch_lo)) return;
     const CloudView& cv = a.cv;
     const GridParams& g = wg.g;
     const int fetch = wg.fetch;
     const int k = wg.k;
-    // LDS: per-wave neighbor lists (features mode), then per wave a 64-entry
-    // compaction scratch of 16 bytes per entry and a 64-entry pending list.
-    const size_t list_words = a.mode != 0 ? 0 : static_cast<size_t>(kWaves) * Q * a.lds_stride;
-    uint32_t* nbr = s_lds + static_cast<size_t>(w) * Q * a.lds_stride;  // lds_stride >= k
-    uint32_t* scratch = s_lds + list_words + static_cast<size_t>(w) * kScratchWords;
-    uint32_t* pending = scratch + 512;  // queries left for the growing search
-    int npend = 0;
+    // LDS: a 64-entry compaction scratch of 16 bytes per entry, twice, then
+    // (features) the queries' neighbor lists.
+    uint32_t* scratch = s_lds;
+    uint32_t* nbr = s_lds + kScratchWords;
     const uint32_t zmask = (1u << g.bz) - 1u;
 
     uint8_t my_flags = 0;
+    uint64_t left = 0;  // the wave's queries not settled here
     uint64_t cnt[3] = {0, 0, 0};  // search passes, candidates, selections
     int qi = 0;
     int rg_prev = 1;  // box half-width of the previous group (density guess)
     // Features with stride 1 keep each neighborhood as a set: the exact-count
     // selection serves them; lists, and strided neighborhoods, need the
     // (d2, id) order.
-    const bool as_set = a.mode == 0 && wg.stride == 1 && a.tune.set_select != 0;
+    const bool as_set = a.mode == 0 && wg.stride == 1;
     // The previous query's threshold, the first one tried (queries in sorted
     // order are close, with similar neighborhood radii).
     double hint = INFINITY;
@@ -864,7 +1687,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
             const int bw = level ? 2 : 1;
             box = Box{bx0 - rg, bx0 + bw - 1 + rg, by0 - rg, by0 + bw - 1 + rg, zmin - rg,
                       zmax + rg};
-            box_ranges(a, wg, box, 0, lane, lo, len);
+            box_ranges(a, wg, box, 0, lane, static_cast<uint32_t>(a.tune.small_col), lo, len);
             const uint32_t incl = wave_incl_scan_u32(len, lane);
             tot = lane_u32(incl, 63);
             excl = incl - len;
@@ -881,7 +1704,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                 // the one box_ranges chunk this path reads.
                 est = est < 1 ? 1 : (est > 3 ? 3 : est);
             }
-            if (tot > kRegCand) {
+            if (tot > kGroupCand) {
                 if (rg > 1) {
                     rg = min(rg - 1, est);
                     continue;
@@ -899,13 +1722,13 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
             break;
         }
         rg_prev = rg;
-        const bool cached = tot <= kRegCand;
+        const bool cached = tot <= kGroupCand;
 
         // Shared candidates of the group's box, cached in registers.
-        double px[kRegBatches], py[kRegBatches], pz[kRegBatches];
-        uint32_t pid[kRegBatches], pj[kRegBatches];
+        double px[kGroupBatches], py[kGroupBatches], pz[kGroupBatches];
+        uint32_t pid[kGroupBatches], pj[kGroupBatches];
 #pragma unroll
-        for (int b = 0; b < kRegBatches; ++b) {
+        for (int b = 0; b < kGroupBatches; ++b) {
             px[b] = py[b] = pz[b] = 0.0;
             pid[b] = pj[b] = kInfU;
             if (cached && static_cast<uint32_t>(b * 64) < tot) {
@@ -931,9 +1754,9 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                 cnt[0] += 1;
                 cnt[1] += tot;
                 // The candidates' ids and positions are the cache's own.
-                uint64_t cd[kRegBatches];
+                uint64_t cd[kGroupBatches];
 #pragma unroll
-                for (int b = 0; b < kRegBatches; ++b)
+                for (int b = 0; b < kGroupBatches; ++b)
                     cd[b] = (static_cast<uint32_t>(b) * 64u < tot && pj[b] != kInfU)
                                 ? dist_bits(qx, qy, qz, px[b], py[b], pz[b])
                                 : kInfD;
@@ -967,7 +1790,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                         // its own and stores its sorted position there.
                         uint32_t base = 0;
 #pragma unroll
-                        for (int b = 0; b < kRegBatches; ++b) {
+                        for (int b = 0; b < kGroupBatches; ++b) {
                             if (static_cast<uint32_t>(b) >= nbat) break;
                             const bool kept = cd[b] <= E;
                             const uint64_t m = __ballot(kept);
@@ -1004,33 +1827,15 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
                     if (done) finish_query(a, wg, best, false, s, qslot, lane, nbr, my_flags);
                 }
             }
-            if (!done) {
-                // Searched alone after the groups, so the group's register
-                // cache is not live at the same time as the growing search.
-                if (lane == 0)
-                    pending[npend] = static_cast<uint32_t>(qslot) |
-                                     (static_cast<uint32_t>(cached ? rg + 1 : 1) << 8);
-                ++npend;
-            }
+            if (!done) left |= 1ull << qslot;
         }
         qi += gm;
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    for (int p = 0; p < npend; ++p) {
-        const uint32_t word = pending[p];
-        const int qslot = static_cast<int>(word & 0xFFu);
-        const uint64_t s = q0 + qslot;
-        const double qx = lane_value(wx, qslot), qy = lane_value(wy, qslot),
-                     qz = lane_value(wz, qslot);
-        const int qcx = static_cast<int>(cell_coord(qx, g.ox, g.inv_c, g.gx));
-        const int qcy = static_cast<int>(cell_coord(qy, g.oy, g.inv_c, g.gy));
-        const int qcz = static_cast<int>(cell_coord(qz, g.oz, g.inv_cz, g.gz));
-        Ent best;
-        bool incomplete = false;
-        search_single(a, wg, qx, qy, qz, qcx, qcy, qcz, static_cast<int>(word >> 8), lane,
-                      scratch, best, incomplete, cnt);
-        finish_query(a, wg, best, incomplete, s, qslot, lane, nbr, my_flags);
+    if (left) {
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(a.out.nflagged + 3, static_cast<uint32_t>(__popcll(left)));
+        at = lane_u32(at, 0) + lanes_below64(left);
+        if ((left >> lane) & 1ull) a.out.deferred[at] = static_cast<uint32_t>(q0 + lane);
     }
     if (a.out.counters && lane == 0) {
         atomicAdd(a.out.counters + 0, static_cast<unsigned long long>(cnt[0]));
@@ -1045,46 +1850,106 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 
-    // One query per lane: FP64 covariance of its neighbor list (two-pass
-    // mean), stored in sorted order for the eigen/feature kernel.
-    if (lane >= nq) return;
+    // One query per lane: FP64 covariance of its neighbor list.
+    if (lane >= nq || ((left >> lane) & 1ull)) return;
     const uint64_t s = q0 + lane;
     const uint32_t* list = nbr + lane * a.lds_stride;
-    // Coordinates relative to the query point (exact differences at any
-    // offset), so the mean carries no rounding of the cloud's absolute
-    // position: at UTM scale that rounding (~1e-9 m) would add a rank-one
-    // term to the covariance of flat and collinear neighborhoods.
-    const double ox = cv.sx[s], oy = cv.sy[s], oz = cv.sz[s];
-    double mx = 0.0, my = 0.0, mz = 0.0;
-    for (int l = 0; l < k; ++l) {
-        const uint32_t j = list[l];
-        mx += cv.sx[j] - ox;
-        my += cv.sy[j] - oy;
-        mz += cv.sz[j] - oz;
-    }
-    mx /= static_cast<double>(k);
-    my /= static_cast<double>(k);
-    mz /= static_cast<double>(k);
-    double c[6] = {0, 0, 0, 0, 0, 0};
-    for (int l = 0; l < k; ++l) {
-        const uint32_t j = list[l];
-        const double dx = (cv.sx[j] - ox) - mx, dy = (cv.sy[j] - oy) - my,
-                     dz = (cv.sz[j] - oz) - mz;
-        c[0] += dx * dx;
-        c[1] += dx * dy;
-        c[2] += dx * dz;
-        c[3] += dy * dy;
-        c[4] += dy * dz;
-        c[5] += dz * dz;
-    }
-    const double den = static_cast<double>(k - 1);
-    double* rec = a.out.cov + kCovRecord * s;
-    for (int i = 0; i < 6; ++i) rec[i] = c[i] / den;
-    reinterpret_cast<uint64_t*>(rec)[6] = my_flags;
+    write_cov_record(a, s, k, wx, wy, wz, my_flags, cv.sx, cv.sy, cv.sz,
+                     [&](int l) { return list[l]; });
     if (my_flags) {
-        uint32_t slot = atomicAdd(a.out.nflagged, 1u);
+        const uint32_t slot = atomicAdd(a.out.nflagged, 1u);
         a.out.flagged[slot] = static_cast<uint32_t>(s);
-        atomicAdd(a.out.nflagged + ((my_flags & ST_INCOMPLETE) ? 2 : 1), 1u);
+        atomicAdd(a.out.nflagged + 1, 1u);
+    }
+}
+
+// The first box of a row's growing search: as many cells to each side as the
+// 3 x 3 x 3 cells around it, taken as a sample of a surface and of a volume,
+// ask for.
+__device__ __forceinline__ int first_ring(const KnnArgs& a, const WaveGrid& wg, int cx, int cy,
+                                          int cz, int lane)
+{
+    const Box b{cx - 1, cx + 1, cy - 1, cy + 1, cz - 1, cz + 1};
+    uint32_t lo, len;
+    box_ranges(a, wg, b, 0, lane, 0u, lo, len);
+    const uint32_t n = lane_u32(wave_incl_scan_u32(len, lane), 63);
+    const float c = static_cast<float>(wg.g.c), h = static_cast<float>(wg.g.cz);
+    const float per = static_cast<float>(wg.fetch + 1) / static_cast<float>(max(n, 1u));
+    const float r = fmaxf(sqrtf(per * 9.0f * c * c * 0.31830989f),
+                          cbrtf(per * 27.0f * c * c * h * 0.23873241f));
+    const float ring = ceilf(1.1f * r / fminf(c, h));
+    return max(a.tune.ring0, min(static_cast<int>(fminf(ring, 1e6f)), min(4, a.tune.ring_max)));
+}
+
+// The rows the lane-per-query search left (out.deferred, their count read on
+// the device), or every row (tuning "set_select" 0): one wave per row with
+// the growing search, kRestRows rows per wave so that the covariances of
+// several rows share their passes.
+constexpr int kRestRows = 4;
+
+template <bool kTiled>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_knn_rest(KnnArgs a)
+{
+    extern __shared__ uint32_t s_lds[];
+    const int lane = __lane_id();
+    uint32_t* scratch = s_lds;
+    uint32_t* nbr = s_lds + kScratchWords;
+    const uint64_t total = a.all_rows ? a.cv.n : a.out.nflagged[3];
+    uint64_t cnt[3] = {0, 0, 0};  // search passes, candidates, selections
+    uint64_t nrows = 0;
+    for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kRestRows; base < total;
+         base += static_cast<uint64_t>(gridDim.x) * kRestRows) {
+        const int nq = static_cast<int>(total - base < kRestRows ? total - base : kRestRows);
+        uint8_t my_flags = 0;
+        uint64_t my_s = 0;
+        int my_k = 0;
+        for (int p = 0; p < nq; ++p) {
+            const uint64_t s = a.all_rows ? base + p : a.out.deferred[base + p];
+            WaveGrid wg;
+            if (kTiled) {
+                const TileInfo& ti = a.tiles[tile_of(a.starts, a.ntiles, s)];
+                if (ti.all_exact) continue;
+                tile_grid(a, ti, wg);
+            } else {
+                cloud_grid(a, wg);
+            }
+            const GridParams& g = wg.g;
+            const double qx = a.cv.sx[s], qy = a.cv.sy[s], qz = a.cv.sz[s];
+            const int qcx = uniform_i32(static_cast<int>(cell_coord(qx, g.ox, g.inv_c, g.gx)));
+            const int qcy = uniform_i32(static_cast<int>(cell_coord(qy, g.oy, g.inv_c, g.gy)));
+            const int qcz = uniform_i32(static_cast<int>(cell_coord(qz, g.oz, g.inv_cz, g.gz)));
+            Ent best;
+            bool incomplete = false;
+            search_single(a, wg, qx, qy, qz, qcx, qcy, qcz, first_ring(a, wg, qcx, qcy, qcz, lane),
+                          lane, scratch, best, incomplete, cnt);
+            finish_query(a, wg, best, incomplete, s, p, lane, nbr, my_flags);
+            if (lane == p) {
+                my_s = s;
+                my_k = wg.k;
+            }
+            nrows += 1;
+        }
+        if (a.mode != 0) continue;
+        // The lists were written by other lanes of this same wave.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < nq && my_k > 0) {
+            const uint32_t* list = nbr + lane * a.lds_stride;
+            write_cov_record(a, my_s, my_k, a.cv.sx[my_s], a.cv.sy[my_s], a.cv.sz[my_s], my_flags,
+                             a.cv.sx, a.cv.sy, a.cv.sz, [&](int l) { return list[l]; });
+            if (my_flags) {
+                const uint32_t slot = atomicAdd(a.out.nflagged, 1u);
+                a.out.flagged[slot] = static_cast<uint32_t>(my_s);
+                atomicAdd(a.out.nflagged + ((my_flags & ST_INCOMPLETE) ? 2 : 1), 1u);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (a.out.counters && lane == 0 && nrows) {
+        atomicAdd(a.out.counters + 0, static_cast<unsigned long long>(cnt[0]));
+        atomicAdd(a.out.counters + 1, static_cast<unsigned long long>(cnt[1]));
+        atomicAdd(a.out.counters + 2, static_cast<unsigned long long>(cnt[2]));
     }
 }
 
@@ -1114,15 +1979,15 @@ struct RadiusArgs {
 };
 
 // Candidates of one chunk: d2 bits per register batch (kInfD outside r).
-__device__ __forceinline__ void radius_pass1(const double (&px)[kRegBatches],
-                                             const double (&py)[kRegBatches],
-                                             const double (&pz)[kRegBatches],
-                                             const uint32_t (&pj)[kRegBatches], uint32_t n1,
+__device__ __forceinline__ void radius_pass1(const double (&px)[kRadBatches],
+                                             const double (&py)[kRadBatches],
+                                             const double (&pz)[kRadBatches],
+                                             const uint32_t (&pj)[kRadBatches], uint32_t n1,
                                              double qx, double qy, double qz, double r2,
                                              uint32_t& cnt, double& sx, double& sy, double& sz)
 {
 #pragma unroll
-    for (int b = 0; b < kRegBatches; ++b) {
+    for (int b = 0; b < kRadBatches; ++b) {
         if (static_cast<uint32_t>(b) * 64u >= n1) break;
         const bool valid = pj[b] != kInfU;
         const double d2 = bits_d2(dist_bits(qx, qy, qz, px[b], py[b], pz[b]));
@@ -1136,15 +2001,15 @@ __device__ __forceinline__ void radius_pass1(const double (&px)[kRegBatches],
     }
 }
 
-__device__ __forceinline__ void radius_pass2(const double (&px)[kRegBatches],
-                                             const double (&py)[kRegBatches],
-                                             const double (&pz)[kRegBatches],
-                                             const uint32_t (&pj)[kRegBatches], uint32_t n1,
+__device__ __forceinline__ void radius_pass2(const double (&px)[kRadBatches],
+                                             const double (&py)[kRadBatches],
+                                             const double (&pz)[kRadBatches],
+                                             const uint32_t (&pj)[kRadBatches], uint32_t n1,
                                              double qx, double qy, double qz, double r2,
                                              double mx, double my, double mz, double (&c)[6])
 {
 #pragma unroll
-    for (int b = 0; b < kRegBatches; ++b) {
+    for (int b = 0; b < kRadBatches; ++b) {
         if (static_cast<uint32_t>(b) * 64u >= n1) break;
         const bool valid = pj[b] != kInfU;
         const double d2 = bits_d2(dist_bits(qx, qy, qz, px[b], py[b], pz[b]));
@@ -1174,7 +2039,6 @@ __global__ __launch_bounds__(256) void k_radius(RadiusArgs a)
     // box_ranges reads only these fields of the kNN arguments.
     KnnArgs ka{};
     ka.cv = cv;
-    ka.tune.small_col = 0;
     WaveGrid wg{};
     wg.g = g;
     wg.colstart = cv.colstart;
@@ -1205,19 +2069,19 @@ __global__ __launch_bounds__(256) void k_radius(RadiusArgs a)
         uint32_t tot = 0;
         for (int cb = 0; cb < ncb; cb += kWave) {
             uint32_t lo, len;
-            box_ranges(ka, wg, box, cb, lane, lo, len);
+            box_ranges(ka, wg, box, cb, lane, 0u, lo, len);
             tot += lane_u32(wave_incl_scan_u32(len, lane), 63);
         }
-        const bool cached = ncb <= kWave && tot <= kRegCand;
-        double px[kRegBatches], py[kRegBatches], pz[kRegBatches];
-        uint32_t pj[kRegBatches];
+        const bool cached = ncb <= kWave && tot <= kRadCand;
+        double px[kRadBatches], py[kRadBatches], pz[kRadBatches];
+        uint32_t pj[kRadBatches];
         uint32_t lo0 = 0, excl0 = 0;
         if (cached) {
             uint32_t len;
-            box_ranges(ka, wg, box, 0, lane, lo0, len);
+            box_ranges(ka, wg, box, 0, lane, 0u, lo0, len);
             excl0 = wave_incl_scan_u32(len, lane) - len;
 #pragma unroll
-            for (int b = 0; b < kRegBatches; ++b) {
+            for (int b = 0; b < kRadBatches; ++b) {
                 px[b] = py[b] = pz[b] = 0.0;
                 pj[b] = kInfU;
                 if (static_cast<uint32_t>(b * 64) < tot) {
@@ -1256,16 +2120,16 @@ __global__ __launch_bounds__(256) void k_radius(RadiusArgs a)
                 // Streamed: chunks of 64 columns and 256 candidates.
                 for (int cb = 0; cb < ncb; cb += kWave) {
                     uint32_t lo, len;
-                    box_ranges(ka, wg, box, cb, lane, lo, len);
+                    box_ranges(ka, wg, box, cb, lane, 0u, lo, len);
                     const uint32_t incl = wave_incl_scan_u32(len, lane);
                     const uint32_t ctot = lane_u32(incl, 63);
                     const uint32_t excl = incl - len;
-                    for (uint32_t t0 = 0; t0 < ctot; t0 += kRegCand) {
-                        double cx[kRegBatches], cy[kRegBatches], czv[kRegBatches];
-                        uint32_t cj[kRegBatches];
-                        const uint32_t n1 = min(ctot - t0, kRegCand);
+                    for (uint32_t t0 = 0; t0 < ctot; t0 += kRadCand) {
+                        double cx[kRadBatches], cy[kRadBatches], czv[kRadBatches];
+                        uint32_t cj[kRadBatches];
+                        const uint32_t n1 = min(ctot - t0, kRadCand);
 #pragma unroll
-                        for (int b = 0; b < kRegBatches; ++b) {
+                        for (int b = 0; b < kRadBatches; ++b) {
                             cx[b] = cy[b] = czv[b] = 0.0;
                             cj[b] = kInfU;
                             if (static_cast<uint32_t>(b * 64) < n1) {
@@ -1308,20 +2172,6 @@ __global__ __launch_bounds__(256) void k_radius(RadiusArgs a)
 
 // Per sorted row: eigensystem of the stored covariance and every requested
 // stage column, written at the row's original index.
-__device__ __forceinline__ uint32_t tile_of(const uint64_t* __restrict__ starts, uint32_t T,
-                                            uint64_t s)
-{
-    uint32_t lo = 0, hi = T;  // largest t with starts[t] <= s
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (starts[mid] <= s)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
 // One thread per row: by original id (kFeaturesAll, kFeaturesUnflagged: a
 // row whose record carries a search flag is skipped), or the i-th row of
 // out.flagged by sorted position (kFeaturesFlagged).
@@ -1420,50 +2270,86 @@ __global__ __launch_bounds__(256) void k_eigen_batch(const double* __restrict__ 
 
 } // namespace
 
+// The search kernels that serve a result capacity.  List entries and kept
+// entries of the query-per-lane instances follow it; above kLaneMaxFetch
+// their registers would not leave two waves per SIMD, and the wave-per-query
+// search serves.
+constexpr int kLaneMaxFetch = 37;
+
+static int lane_class(int fetch)
+{
+    return fetch <= 9 ? 0 : fetch <= 21 ? 1 : fetch <= kLaneMaxFetch ? 2 : 3;
+}
+
+uint32_t knn_class_bit(int fetch) { return 1u << lane_class(fetch); }
+
+template <bool kTiled>
+static void launch_lane(KnnArgs& a, uint32_t classes, uint32_t blocks, hipStream_t s)
+{
+    bool again = false;
+    auto one = [&](uint32_t bit, int lo, int hi, auto lane, auto pair) {
+        if (!(classes & bit)) return;
+        if (again) {  // the heavy list starts over with each class
+            launch_fill_u32(a.out.nflagged + 4, 1, 0u, s);
+            launch_fill_u32(a.out.nflagged + 7, 1, 0u, s);
+        }
+        again = true;
+        a.fetch_lo = lo;
+        a.fetch_hi = hi;
+        hipLaunchKernelGGL(lane, dim3(blocks), dim3(64), 0, s, a);
+        hipLaunchKernelGGL(pair, dim3(std::min<uint32_t>(2 * blocks, 2048)), dim3(64), 0, s, a);
+    };
+    one(1u, 0, 9, k_knn_lane<24, 12, 2, kTiled>, k_knn_pair<20, 12, 2, kTiled>);
+    one(2u, 10, 21, k_knn_lane<40, 24, 2, kTiled>, k_knn_pair<32, 24, 2, kTiled>);
+    one(4u, 22, kLaneMaxFetch, k_knn_lane<56, 40, 2, kTiled>, k_knn_pair<48, 40, 2, kTiled>);
+    if (classes & 8u) {
+        a.fetch_lo = kLaneMaxFetch + 1;
+        a.fetch_hi = kMaxFetch - 1;
+        const size_t lds = (kScratchWords + (a.mode != 0 ? 0 : a.q_per_wave * a.lds_stride)) *
+                           sizeof(uint32_t);
+        hipLaunchKernelGGL(k_knn_group<kTiled>, dim3(blocks), dim3(64), lds, s, a);
+    }
+}
+
 void launch_knn(const CloudView& cv, const FusedProgram& prog, int mode,
                 const KnnOutputs& out, const KnnTuning& tune, hipStream_t s,
                 const TileTables* tt)
 {
     if (cv.n == 0) return;
-    KnnArgs a;
+    KnnArgs a{};
     a.cv = cv;
     a.prog = prog;
     a.out = out;
     a.tune = tune;
     a.mode = mode;
-    a.tiles = nullptr;
-    a.task0 = nullptr;
-    a.ntasks = 0;
-    a.ntiles = 0;
+    a.all_rows = tune.set_select ? 0 : 1;
     const int max_k = tt ? tt->max_k : prog.k;
     a.q_per_wave = tt ? tt->q_per_wave
-                      : (tune.q_per_wave > 0 ? tune.q_per_wave : knn_queries_per_wave(prog.k));
+                      : (tune.q_per_wave > 0 ? tune.q_per_wave : kQueriesPerWave);
     a.lds_stride = max_k | 1;  // odd stride: lanes hit distinct LDS banks
     const GridParams& g = cv.g;
     a.margin = 1e-6 * fmin(g.c, g.cz) +
                1e-15 * (fabs(g.ox) + fabs(g.oy) + fabs(g.oz)) + 1e-300;
-    const int wv = tune.waves == 1 || tune.waves == 2 ? tune.waves : kKnnWavesDefault;
-    const size_t waves = static_cast<size_t>(tt ? 1 : wv);
-    const size_t list_words = mode != 0 ? 0 : waves * a.q_per_wave * a.lds_stride;
-    const size_t lds = (list_words + waves * kScratchWords) * sizeof(uint32_t);
+    // The rest: a grid for the few rows usually left (one wave per kRestRows
+    // of them; the kernel walks any number).
+    const uint32_t rest = static_cast<uint32_t>(std::min<uint64_t>(
+        div_up(cv.n, kRestRows), a.all_rows ? 65536u : 8192u));
+    const size_t lds = (kScratchWords + (mode != 0 ? 0 : kRestRows * a.lds_stride)) *
+                       sizeof(uint32_t);
     if (tt) {
         if (!tt->ntasks) return;
         a.tiles = tt->tiles;
+        a.starts = tt->starts;
         a.task0 = tt->task0;
         a.ntasks = tt->ntasks;
         a.ntiles = tt->ntiles;
-        const uint32_t blocks = div_up(tt->ntasks, waves);
-        hipLaunchKernelGGL((k_knn<true, 1>), dim3(blocks), dim3(waves * kWave), lds, s, a);
+        if (!a.all_rows) launch_lane<true>(a, tt->classes, tt->ntasks, s);
+        hipLaunchKernelGGL(k_knn_rest<true>, dim3(rest), dim3(64), lds, s, a);
         return;
     }
-    const uint64_t per_block = static_cast<uint64_t>(waves) * a.q_per_wave;
-    const uint32_t blocks = div_up(cv.n, per_block);
-    if (wv == 1)
-        hipLaunchKernelGGL((k_knn<false, 1>), dim3(blocks), dim3(waves * kWave), lds, s, a);
-    else if (wv == 2)
-        hipLaunchKernelGGL((k_knn<false, 2>), dim3(blocks), dim3(waves * kWave), lds, s, a);
-    else
-        hipLaunchKernelGGL((k_knn<false, 4>), dim3(blocks), dim3(waves * kWave), lds, s, a);
+    if (!a.all_rows)
+        launch_lane<false>(a, knn_class_bit(prog.fetch), div_up(cv.n, a.q_per_wave), s);
+    hipLaunchKernelGGL(k_knn_rest<false>, dim3(rest), dim3(64), lds, s, a);
 }
 
 void launch_radius(const CloudView& cv, double radius, int mode, double* cov, uint32_t* counts,
