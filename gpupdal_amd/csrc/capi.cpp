@@ -533,7 +533,8 @@ void Context::run_group_radius(Cloud& cl, const gf_stage* st, int ns, double* co
     out.cov = covbuf.as<double>();
     const CloudView cv = view(cl);
     hipEvent_t e0 = mark();
-    launch_radius(cv, r, 0, out.cov, nullptr, tune.group_z, stream);
+    flagged.ensure((n + 1) * 4);
+    launch_radius(cv, r, 0, out.cov, nullptr, flagged.as<uint32_t>(), stream);
     hipEvent_t e1 = mark();
     span(e0, e1, &stats.ms_search);
     launch_features(cv, prog, out, cl.inv.as<uint32_t>(), stream, nullptr, kFeaturesAll);
@@ -1121,7 +1122,8 @@ int gf_radius_counts(gf_ctx* ctx, gf_cloud* cloud, double radius, uint32_t* coun
             c->outbuf.ensure(n * 4 + 8);
             dst = c->outbuf.as<uint32_t>();
         }
-        launch_radius(c->view(*cl), radius, 1, nullptr, dst, c->tune.group_z, c->stream);
+        c->flagged.ensure((n + 1) * 4);
+        launch_radius(c->view(*cl), radius, 1, nullptr, dst, c->flagged.as<uint32_t>(), c->stream);
         if (where == GF_WHERE_HOST)
             GF_HIP(hipMemcpyAsync(counts, dst, n * 4, hipMemcpyDeviceToHost, c->stream));
         GF_HIP(hipStreamSynchronize(c->stream));
@@ -1201,8 +1203,9 @@ int gf_outlier(gf_ctx* ctx, gf_cloud* cloud, int method, uint32_t mean_k, double
             c->points_mark = false;
             c->build_index(*cl, 0, radius * c->tune.radius_cell);
             c->outbuf.ensure(n * 4 + 8);
+            c->flagged.ensure((n + 1) * 4);
             launch_radius(c->view(*cl), radius, 1, nullptr, c->outbuf.as<uint32_t>(),
-                          c->tune.group_z, c->stream);
+                          c->flagged.as<uint32_t>(), c->stream);
             std::vector<uint32_t> counts(n);
             GF_HIP(hipMemcpyAsync(counts.data(), c->outbuf.ptr, n * 4, hipMemcpyDeviceToHost,
                                   c->stream));

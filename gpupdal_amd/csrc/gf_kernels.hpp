@@ -120,7 +120,7 @@ struct KnnTuning {
     int32_t ring0;       // first ring (box half-width in columns)
     int32_t ring_max;    // budget before a row is marked incomplete
     int32_t small_col;   // columns up to this size are taken whole
-    int32_t group_z;     // radius search: z cells beyond the first a query group may span
+    int32_t group_z;     // wave-per-query search: z cells beyond the first a query group may span
     int32_t q_per_wave;  // queries per wave (0: by the number of points)
     int32_t set_select;  // 1: lane-per-query search; 0: every row by the growing search
 };
@@ -211,9 +211,10 @@ void launch_knn(const CloudView& cv, const FusedProgram& prog, int mode,
                 const TileTables* tt = nullptr);
 // Radius neighborhoods: mode 0 writes each sorted row's covariance record
 // (FP64 two-pass over the points with d2 < radius^2, neighbor count in word
-// 7); mode 1 writes the counts (original order) to `counts`.
+// 7); mode 1 writes the counts (original order) to `counts`.  rest: n + 1
+// words of working space.
 void launch_radius(const CloudView& cv, double radius, int mode, double* cov, uint32_t* counts,
-                   int group_z, hipStream_t s);
+                   uint32_t* rest, hipStream_t s);
 // Eigensystem + stage columns from out.cov, in original point order (inv:
 // original id -> sorted position), so outputs are written contiguously.
 // rows: kFeaturesAll every row; kFeaturesUnflagged every row the search did

@@ -68,7 +68,7 @@ struct Tuning {
     int ring0 = 1;
     int ring_max = 8;
     int small_col = 0;
-    int group_z = 3;             // radius search: z cells a query group may span
+    int group_z = 3;             // wave-per-query search: z cells a query group may span
     int q_per_wave = 0;          // queries per search wave (0: 64)
     int knn_waves = 0;           // accepted, without effect: the search's workgroups are waves
     int set_select = 1;          // 1: query-per-lane search; 0: every row by the growing search

@@ -994,6 +994,7 @@ __device__ __forceinline__ void load_sorted(const uint32_t* my, uint32_t cnt, ui
 }
 
 template <int CAP> struct StageShared {
+    static constexpr bool kPositions = true;
     double x[kStageMax], y[kStageMax], z[kStageMax];
     uint32_t j[kStageMax];
     uint32_t cell[kStageCells + 2];   // counts, then first slots; last: points left out
@@ -1007,6 +1008,118 @@ __device__ __forceinline__ void wave_lds_order()
 {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+
+// A box staged in LDS: its faces and its cells (counts and 1 / edges).
+struct StageBox {
+    double X0 = 0, X1 = 0, Y0 = 0, Y1 = 0, Z0 = 0, Z1 = 0;
+    float hx = 0, hy = 0, hz = 0;
+    int nx = 1, ny = 1, nz = 1;
+};
+
+// Stages the points of N <= kStageRaw column entries (lo, len: the lane's
+// columns; at: entries of the lanes before it) that lie inside B's faces,
+// counting-sorted by cell.  False if there are more than kStageMax.
+template <class Shared>
+__device__ __forceinline__ bool stage_points(const CloudView& cv, Shared& S,
+                                             const uint32_t (&lo)[kStageCols],
+                                             const uint32_t (&len)[kStageCols], uint32_t at,
+                                             uint32_t N, const StageBox& B, int lane)
+{
+    // The columns' points, one per lane and slot.
+#pragma unroll
+    for (int i = 0; i < kStageCols; ++i)
+        for (uint32_t c = 0; c < len[i]; ++c) S.pos[at++] = lo[i] + c;
+#pragma unroll
+    for (uint32_t c = 0; c < kStageCells; c += 64) S.cell[c + lane] = 0;
+    wave_lds_order();
+    // Four points per lane at a time; the coordinates are read
+    // again (from cache) when the slots are known, so that
+    // they do not hold registers in between.
+    uint32_t pc[kStageSlots];  // cell << 16 | rank in it, or ~0
+#pragma unroll
+    for (int i0 = 0; i0 < kStageSlots; i0 += 4) {
+        if (i0 * 64u >= N) {  // wave-uniform
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pc[i0 + i] = ~0u;
+            continue;
+        }
+        double px[4], py[4], pz[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t t = (i0 + i) * 64u + lane;
+            const uint32_t j = S.pos[t < N ? t : 0u];
+            px[i] = cv.sx[j];
+            py[i] = cv.sy[j];
+            pz[i] = cv.sz[j];
+        }
+        uint32_t cell[4], rank[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t t = (i0 + i) * 64u + lane;
+            const int ix = min(static_cast<int>(static_cast<float>(px[i] - B.X0) * B.hx), B.nx - 1);
+            const int iy = min(static_cast<int>(static_cast<float>(py[i] - B.Y0) * B.hy), B.ny - 1);
+            const int iz = min(static_cast<int>(static_cast<float>(pz[i] - B.Z0) * B.hz), B.nz - 1);
+            const bool in = static_cast<int>(t < N) & static_cast<int>(px[i] >= B.X0) &
+                            static_cast<int>(px[i] <= B.X1) & static_cast<int>(py[i] >= B.Y0) &
+                            static_cast<int>(py[i] <= B.Y1) & static_cast<int>(pz[i] >= B.Z0) &
+                            static_cast<int>(pz[i] <= B.Z1);
+            // (points outside count in a cell of their own)
+            cell[i] = in ? static_cast<uint32_t>((iz * B.ny + iy) * B.nx + ix) : kStageCells + 1u;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rank[i] = atomicAdd(&S.cell[cell[i]], 1u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            pc[i0 + i] = cell[i] <= kStageCells ? (cell[i] << 16) | rank[i] : ~0u;
+    }
+    wave_lds_order();
+    // First slots of the cells (eight cells per lane).
+    constexpr int kPer = kStageCells / 64;
+    uint32_t v[kPer], sum = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        v[i] = S.cell[lane * kPer + i];
+        sum += v[i];
+    }
+    uint32_t ex = wave_scan_u32(sum);
+    const uint32_t M = lane_u32(ex, 63);
+    ex -= sum;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        S.cell[lane * kPer + i] = ex;
+        ex += v[i];
+    }
+    if (lane == 0) S.cell[kStageCells] = M;
+    wave_lds_order();
+    if (M > kStageMax) return false;
+#pragma unroll
+    for (int i0 = 0; i0 < kStageSlots; i0 += 4) {
+        if (i0 * 64u >= N) break;
+        double px[4], py[4], pz[4];
+        uint32_t j[4], at[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t t = (i0 + i) * 64u + lane;
+            j[i] = S.pos[t < N ? t : 0u];
+            px[i] = cv.sx[j[i]];
+            py[i] = cv.sy[j[i]];
+            pz[i] = cv.sz[j[i]];
+            const uint32_t c = pc[i0 + i];
+            at[i] = c != ~0u ? S.cell[c >> 16] + (c & 0xFFFFu) : ~0u;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (at[i] != ~0u) {
+                S.x[at[i]] = px[i];
+                S.y[at[i]] = py[i];
+                S.z[at[i]] = pz[i];
+                if constexpr (Shared::kPositions) S.j[at[i]] = j[i];
+            }
+        }
+    }
+    wave_lds_order();
+    return true;
 }
 
 // FP64 covariance of the k neighbors pos(0..k-1) (indexes into x, y, z;
@@ -1166,9 +1279,7 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
         const uint32_t first_tries = lane_u32(tries, first);
         bool act = pending && tries == first_tries;
         float r = r_first;
-        double X0 = 0, X1 = 0, Y0 = 0, Y1 = 0, Z0 = 0, Z1 = 0;
-        float hx = 0, hy = 0, hz = 0;  // 1 / cell edges of the staged box
-        int nx = 1, ny = 1, nz = 1;
+        StageBox B;
         bool got = false;
         int refine = 0;
         for (int step = 0; step < 16; ++step) {
@@ -1181,20 +1292,20 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
             // rounding and the FP64 rounding of the faces taken off.
             const float W = fmaxf(fmaxf(fmaxf(-lx, ux), fmaxf(-ly, uy)), fmaxf(-lz, uz)) + r;
             const double pad = static_cast<double>(r) + 3e-7 * static_cast<double>(W) + wg.margin;
-            X0 = bx + static_cast<double>(lx) - pad;
-            X1 = bx + static_cast<double>(ux) + pad;
-            Y0 = by + static_cast<double>(ly) - pad;
-            Y1 = by + static_cast<double>(uy) + pad;
-            Z0 = bz + static_cast<double>(lz) - pad;
-            Z1 = bz + static_cast<double>(uz) + pad;
+            B.X0 = bx + static_cast<double>(lx) - pad;
+            B.X1 = bx + static_cast<double>(ux) + pad;
+            B.Y0 = by + static_cast<double>(ly) - pad;
+            B.Y1 = by + static_cast<double>(uy) + pad;
+            B.Z0 = bz + static_cast<double>(lz) - pad;
+            B.Z1 = bz + static_cast<double>(uz) + pad;
             // Grid cells by the points' own rule, so that a point inside the
             // faces is inside the cells.
-            const Box b{uniform_i32(static_cast<int>(cell_coord(X0, g.ox, g.inv_c, g.gx))),
-                        uniform_i32(static_cast<int>(cell_coord(X1, g.ox, g.inv_c, g.gx))),
-                        uniform_i32(static_cast<int>(cell_coord(Y0, g.oy, g.inv_c, g.gy))),
-                        uniform_i32(static_cast<int>(cell_coord(Y1, g.oy, g.inv_c, g.gy))),
-                        uniform_i32(static_cast<int>(cell_coord(Z0, g.oz, g.inv_cz, g.gz))),
-                        uniform_i32(static_cast<int>(cell_coord(Z1, g.oz, g.inv_cz, g.gz)))};
+            const Box b{uniform_i32(static_cast<int>(cell_coord(B.X0, g.ox, g.inv_c, g.gx))),
+                        uniform_i32(static_cast<int>(cell_coord(B.X1, g.ox, g.inv_c, g.gx))),
+                        uniform_i32(static_cast<int>(cell_coord(B.Y0, g.oy, g.inv_c, g.gy))),
+                        uniform_i32(static_cast<int>(cell_coord(B.Y1, g.oy, g.inv_c, g.gy))),
+                        uniform_i32(static_cast<int>(cell_coord(B.Z0, g.oz, g.inv_cz, g.gz))),
+                        uniform_i32(static_cast<int>(cell_coord(B.Z1, g.oz, g.inv_cz, g.gz)))};
             const uint64_t ncb = static_cast<uint64_t>(b.x1 - b.x0 + 1) *
                                  static_cast<uint64_t>(b.y1 - b.y0 + 1);
             bool over = ncb > kStageCols * 64u;
@@ -1226,117 +1337,22 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
                     // Cells: a third of the radius along x (runs are cut
                     // there), half of it along y, the radius along z when the
                     // box is tall.
-                    const float Lx = static_cast<float>(X1 - X0), Ly = static_cast<float>(Y1 - Y0),
-                                Lz = static_cast<float>(Z1 - Z0);
+                    const float Lx = static_cast<float>(B.X1 - B.X0), Ly = static_cast<float>(B.Y1 - B.Y0),
+                                Lz = static_cast<float>(B.Z1 - B.Z0);
                     float cx = r * 0.34f, cy = r * 0.5f, cz = r;
                     for (;;) {
-                        nx = uniform_i32(static_cast<int>(fminf(Lx / cx, 1000.0f)) + 1);
-                        ny = uniform_i32(static_cast<int>(fminf(Ly / cy, 1000.0f)) + 1);
-                        nz = uniform_i32(Lz > 4.0f * r ? static_cast<int>(fminf(Lz / cz, 1000.0f)) + 1 : 1);
-                        if (static_cast<uint32_t>(nx * ny * nz) <= kStageCells) break;
+                        B.nx = uniform_i32(static_cast<int>(fminf(Lx / cx, 1000.0f)) + 1);
+                        B.ny = uniform_i32(static_cast<int>(fminf(Ly / cy, 1000.0f)) + 1);
+                        B.nz = uniform_i32(Lz > 4.0f * r ? static_cast<int>(fminf(Lz / cz, 1000.0f)) + 1 : 1);
+                        if (static_cast<uint32_t>(B.nx * B.ny * B.nz) <= kStageCells) break;
                         cx *= 1.3f;
                         cy *= 1.3f;
                         cz *= 1.3f;
                     }
-                    hx = 1.0f / cx;
-                    hy = 1.0f / cy;
-                    hz = nz > 1 ? 1.0f / cz : 0.0f;
-                    // The columns' points, one per lane and slot.
-                    uint32_t at = incl - part;
-#pragma unroll
-                    for (int i = 0; i < kStageCols; ++i)
-                        for (uint32_t c = 0; c < len[i]; ++c) S.pos[at++] = lo[i] + c;
-#pragma unroll
-                    for (uint32_t c = 0; c < kStageCells; c += 64) S.cell[c + lane] = 0;
-                    wave_lds_order();
-                    // Four points per lane at a time; the coordinates are read
-                    // again (from cache) when the slots are known, so that
-                    // they do not hold registers in between.
-                    uint32_t pc[kStageSlots];  // cell << 16 | rank in it, or ~0
-#pragma unroll
-                    for (int i0 = 0; i0 < kStageSlots; i0 += 4) {
-                        if (i0 * 64u >= N) {  // wave-uniform
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) pc[i0 + i] = ~0u;
-                            continue;
-                        }
-                        double px[4], py[4], pz[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const uint32_t t = (i0 + i) * 64u + lane;
-                            const uint32_t j = S.pos[t < N ? t : 0u];
-                            px[i] = cv.sx[j];
-                            py[i] = cv.sy[j];
-                            pz[i] = cv.sz[j];
-                        }
-                        uint32_t cell[4], rank[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const uint32_t t = (i0 + i) * 64u + lane;
-                            const int ix = min(static_cast<int>(static_cast<float>(px[i] - X0) * hx), nx - 1);
-                            const int iy = min(static_cast<int>(static_cast<float>(py[i] - Y0) * hy), ny - 1);
-                            const int iz = min(static_cast<int>(static_cast<float>(pz[i] - Z0) * hz), nz - 1);
-                            const bool in = static_cast<int>(t < N) & static_cast<int>(px[i] >= X0) &
-                                            static_cast<int>(px[i] <= X1) & static_cast<int>(py[i] >= Y0) &
-                                            static_cast<int>(py[i] <= Y1) & static_cast<int>(pz[i] >= Z0) &
-                                            static_cast<int>(pz[i] <= Z1);
-                            // (points outside count in a cell of their own)
-                            cell[i] = in ? static_cast<uint32_t>((iz * ny + iy) * nx + ix) : kStageCells + 1u;
-                        }
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) rank[i] = atomicAdd(&S.cell[cell[i]], 1u);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            pc[i0 + i] = cell[i] <= kStageCells ? (cell[i] << 16) | rank[i] : ~0u;
-                    }
-                    wave_lds_order();
-                    // First slots of the cells (eight cells per lane).
-                    constexpr int kPer = kStageCells / 64;
-                    uint32_t v[kPer], sum = 0;
-#pragma unroll
-                    for (int i = 0; i < kPer; ++i) {
-                        v[i] = S.cell[lane * kPer + i];
-                        sum += v[i];
-                    }
-                    uint32_t ex = wave_scan_u32(sum);
-                    const uint32_t M = lane_u32(ex, 63);
-                    ex -= sum;
-#pragma unroll
-                    for (int i = 0; i < kPer; ++i) {
-                        S.cell[lane * kPer + i] = ex;
-                        ex += v[i];
-                    }
-                    if (lane == 0) S.cell[kStageCells] = M;
-                    wave_lds_order();
-                    over = M > kStageMax;
-                    if (!over) {
-#pragma unroll
-                        for (int i0 = 0; i0 < kStageSlots; i0 += 4) {
-                            if (i0 * 64u >= N) break;
-                            double px[4], py[4], pz[4];
-                            uint32_t j[4], at[4];
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                const uint32_t t = (i0 + i) * 64u + lane;
-                                j[i] = S.pos[t < N ? t : 0u];
-                                px[i] = cv.sx[j[i]];
-                                py[i] = cv.sy[j[i]];
-                                pz[i] = cv.sz[j[i]];
-                                const uint32_t c = pc[i0 + i];
-                                at[i] = c != ~0u ? S.cell[c >> 16] + (c & 0xFFFFu) : ~0u;
-                            }
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                if (at[i] != ~0u) {
-                                    S.x[at[i]] = px[i];
-                                    S.y[at[i]] = py[i];
-                                    S.z[at[i]] = pz[i];
-                                    S.j[at[i]] = j[i];
-                                }
-                            }
-                        }
-                        wave_lds_order();
-                    }
+                    B.hx = 1.0f / cx;
+                    B.hy = 1.0f / cy;
+                    B.hz = B.nz > 1 ? 1.0f / cz : 0.0f;
+                    over = !stage_points(cv, S, lo, len, incl - part, N, B, lane);
                 }
             }
             if (!over) {
@@ -1361,18 +1377,18 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
         // The lane's cells at radius rl: rows and layers [*0, *1].
         float rl = r;
         int cx0 = 0, cx1 = 0, cy0 = 0, cy1 = -1, cz0 = 0, cz1 = 0;
-        const float fx = static_cast<float>(qx - X0), fy = static_cast<float>(qy - Y0),
-                    fz = static_cast<float>(qz - Z0);
+        const float fx = static_cast<float>(qx - B.X0), fy = static_cast<float>(qy - B.Y0),
+                    fz = static_cast<float>(qz - B.Z0);
         auto cells = [&](float rr) {
             // A hair wider than rr, so that rounding loses no point.
             const float e = rr * 1.0001f + 1e-6f * (fabsf(fx) + fabsf(fy) + fabsf(fz)) +
                             static_cast<float>(wg.margin);
-            cx0 = min(static_cast<int>(fmaxf(fx - e, 0.0f) * hx), nx - 1);
-            cx1 = min(static_cast<int>((fx + e) * hx), nx - 1);
-            cy0 = static_cast<int>(fmaxf(fy - e, 0.0f) * hy);
-            cy1 = act ? min(static_cast<int>((fy + e) * hy), ny - 1) : cy0 - 1;
-            cz0 = min(static_cast<int>(fmaxf(fz - e, 0.0f) * hz), nz - 1);
-            cz1 = act ? min(static_cast<int>((fz + e) * hz), nz - 1) : cz0 - 1;
+            cx0 = min(static_cast<int>(fmaxf(fx - e, 0.0f) * B.hx), B.nx - 1);
+            cx1 = min(static_cast<int>((fx + e) * B.hx), B.nx - 1);
+            cy0 = static_cast<int>(fmaxf(fy - e, 0.0f) * B.hy);
+            cy1 = act ? min(static_cast<int>((fy + e) * B.hy), B.ny - 1) : cy0 - 1;
+            cz0 = min(static_cast<int>(fmaxf(fz - e, 0.0f) * B.hz), B.nz - 1);
+            cz1 = act ? min(static_cast<int>((fz + e) * B.hz), B.nz - 1) : cz0 - 1;
         };
         cells(r);
         // Where the box is denser around this query than its radius asks for,
@@ -1381,7 +1397,7 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
             uint32_t seen = 0;
             for (int z = cz0; z <= cz1; ++z)
                 for (int y = cy0; y <= cy1; ++y) {
-                    const int row = (z * ny + y) * nx;
+                    const int row = (z * B.ny + y) * B.nx;
                     seen += S.cell[row + cx1 + 1] - S.cell[row + cx0];
                 }
             // At least a quarter of those seen are inside the radius, and
@@ -1403,7 +1419,7 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
             for (int dy = 0; __ballot(cy0 + dy <= cy1); ++dy) {
                 uint32_t p = 0, e = 0;
                 if (cy0 + dy <= cy1 && cz0 + dz <= cz1) {
-                    const int row = ((cz0 + dz) * ny + cy0 + dy) * nx;
+                    const int row = ((cz0 + dz) * B.ny + cy0 + dy) * B.nx;
                     p = S.cell[row + cx0] + part;
                     e = S.cell[row + cx1 + 1];
                     seen += e - p;
@@ -1958,24 +1974,35 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 // pdal/private/KDImpl.hpp:398-415, nanoflann radiusSearch): every point whose
 // FP64 squared distance (KD3Index's operation order) is strictly below r*r.
 // The set is decided by that comparison alone -- no boundary tie, no exact
-// re-solve.  A wavefront takes a group of consecutive sorted queries (one
-// 2x2 block of columns with nearby z cells, as the kNN search groups them)
-// and the box of every cell that can hold a point within r of any of them:
-// the block grown by R = ceil(r / c) columns, the group's z cells by
-// ceil(r / cz) (cell edges chosen so that R is 2).  Per query the
-// wavefront masks the box's candidates by d2 < r*r and forms the count and
-// the FP64 two-pass covariance (coordinates relative to the query point)
-// from masked wavefront sums.  Boxes of up to 256 candidates and 64 columns
-// are held in registers for the whole group; larger boxes are streamed from
-// memory per query.
+// re-solve.  A wave takes 64 spatially compact queries, one per lane, and
+// stages the points of their bounding box grown by r in LDS, sorted into
+// cells, as the kNN search does; each lane walks the runs of cells within r of
+// its query, once for the count and the mean (coordinates relative to the
+// query) and once more for the FP64 covariance about it.  A group whose box
+// holds too many points is halved along its longest axis; where kRadiusFew
+// queries still do not fit, the wave's remaining rows go to k_radius_rest, one
+// wave per row, which streams the row's columns from memory, 256 candidates at
+// a time.
+//
+// Bound by LDS reads and FP64 instructions.  With one row at a time per
+// wavefront, candidates masked by ballots and every covariance entry summed
+// across the wave, 1M points of 28 neighbors (median; 5% above 300) took 7.8
+// ms; now 1.8 ms.
+// kRadiusFew: the search there takes 2.1 ms at 8, 1.88 at 16, 1.81 at 24, 1.78
+// at 33, 1.81 without halving: each halving is one more staging round of a
+// wave, with fewer lanes at work.
+constexpr int kRadiusFew = 32;
+
 struct RadiusArgs {
     CloudView cv;
     double r2;          // r * r, the strict bound on d2
+    float r;            // r, rounded up
+    double margin;      // of the cells' faces
     int32_t rx, rz;     // box growth in columns and z cells
-    int32_t group_z;
     int32_t mode;       // 0: covariance records; 1: counts only
     double* cov;        // mode 0: records in sorted order (count in word 7)
     uint32_t* counts;   // mode 1: counts in original order
+    uint32_t* rest;     // rows left to k_radius_rest: their number, then they
 };
 
 // Candidates of one chunk: d2 bits per register batch (kInfD outside r).
@@ -2025,149 +2052,285 @@ __device__ __forceinline__ void radius_pass2(const double (&px)[kRadBatches],
     }
 }
 
-__global__ __launch_bounds__(256) void k_radius(RadiusArgs a)
+struct RadiusShared {
+    static constexpr bool kPositions = false;
+    double x[kStageMax], y[kStageMax], z[kStageMax];
+    uint32_t j[1];
+    uint32_t cell[kStageCells + 2];
+    uint32_t pos[kStageRaw];
+};
+
+__device__ __forceinline__ void write_radius_row(const RadiusArgs& a, uint64_t s, uint32_t cnt,
+                                                 const double (&c)[6])
 {
-    const int lane = __lane_id();
-    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
-    const uint32_t lb = xcd_logical_block(blockIdx.x, gridDim.x);
+    if (a.mode == 1) {
+        a.counts[a.cv.perm[s]] = cnt;
+        return;
+    }
+    const double den = static_cast<double>(cnt) - 1.0;
+    double* rec = a.cov + kCovRecord * s;
+#pragma unroll
+    for (int i = 0; i < 6; ++i) rec[i] = c[i] / den;
+    reinterpret_cast<uint64_t*>(rec)[6] = 0;
+    reinterpret_cast<uint64_t*>(rec)[7] = cnt;
+}
+
+// One row by the whole wave, streamed from memory.
+__device__ __forceinline__ void radius_row(const RadiusArgs& a, const KnnArgs& ka,
+                                           const WaveGrid& wg, uint64_t s, int lane)
+{
     const CloudView& cv = a.cv;
     const GridParams& g = cv.g;
-    const uint64_t q0 = (static_cast<uint64_t>(lb) * 4 + w) * kWave;
+    const double qx = cv.sx[s], qy = cv.sy[s], qz = cv.sz[s];
+    const int qcx = uniform_i32(static_cast<int>(cell_coord(qx, g.ox, g.inv_c, g.gx)));
+    const int qcy = uniform_i32(static_cast<int>(cell_coord(qy, g.oy, g.inv_c, g.gy)));
+    const int qcz = static_cast<int>(uniform_u32(cv.keys[s]) & ((1u << g.bz) - 1u));
+    const Box box{qcx - a.rx, qcx + a.rx, qcy - a.rx, qcy + a.rx, qcz - a.rz, qcz + a.rz};
+    const int ncb = (1 + 2 * a.rx) * (1 + 2 * a.rx);
+    uint32_t cnt = 0;
+    double sx = 0.0, sy = 0.0, sz = 0.0;
+    double c[6] = {0, 0, 0, 0, 0, 0};
+    for (int pass = 0; pass < (a.mode == 0 ? 2 : 1); ++pass) {
+        double mx = 0.0, my = 0.0, mz = 0.0;
+        if (pass == 1) {
+            const double nn = static_cast<double>(cnt);
+            mx = wave_sum_f64(sx) / nn;
+            my = wave_sum_f64(sy) / nn;
+            mz = wave_sum_f64(sz) / nn;
+        }
+        // Chunks of 64 columns and 256 candidates.
+        for (int cb = 0; cb < ncb; cb += kWave) {
+            uint32_t lo, len;
+            box_ranges(ka, wg, box, cb, lane, 0u, lo, len);
+            const uint32_t incl = wave_incl_scan_u32(len, lane);
+            const uint32_t ctot = lane_u32(incl, 63);
+            const uint32_t excl = incl - len;
+            for (uint32_t t0 = 0; t0 < ctot; t0 += kRadCand) {
+                double cx[kRadBatches], cy[kRadBatches], czv[kRadBatches];
+                uint32_t cj[kRadBatches];
+                const uint32_t n1 = min(ctot - t0, kRadCand);
+#pragma unroll
+                for (int b = 0; b < kRadBatches; ++b) {
+                    cx[b] = cy[b] = czv[b] = 0.0;
+                    cj[b] = kInfU;
+                    if (static_cast<uint32_t>(b * 64) < n1) {
+                        const uint32_t t = t0 + b * 64 + lane;
+                        const uint32_t j = candidate_pos(lo, excl, t);
+                        if (t < ctot) {
+                            cx[b] = cv.sx[j];
+                            cy[b] = cv.sy[j];
+                            czv[b] = cv.sz[j];
+                            cj[b] = j;
+                        }
+                    }
+                }
+                if (pass == 0)
+                    radius_pass1(cx, cy, czv, cj, n1, qx, qy, qz, a.r2, cnt, sx, sy, sz);
+                else
+                    radius_pass2(cx, cy, czv, cj, n1, qx, qy, qz, a.r2, mx, my, mz, c);
+            }
+        }
+    }
+    if (a.mode == 0) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) c[i] = wave_sum_f64(c[i]);
+    }
+    if (lane == 0) write_radius_row(a, s, cnt, c);
+}
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_radius(RadiusArgs a)
+{
+    __shared__ RadiusShared S;
+    const int lane = __lane_id();
+    const CloudView& cv = a.cv;
+    const GridParams& g = cv.g;
+    const uint64_t q0 = static_cast<uint64_t>(xcd_logical_block(blockIdx.x, gridDim.x)) * 64u;
     if (q0 >= cv.n) return;
     const int nq = static_cast<int>(cv.n - q0 < 64 ? cv.n - q0 : 64);
-    const uint32_t zmask = (1u << g.bz) - 1u;
-    // box_ranges reads only these fields of the kNN arguments.
+    // box_ranges and box_columns read only these fields of the kNN arguments.
     KnnArgs ka{};
     ka.cv = cv;
     WaveGrid wg{};
     wg.g = g;
     wg.colstart = cv.colstart;
-    int qi = 0;
-    while (qi < nq) {
-        const uint64_t s0 = q0 + qi;
-        const bool in_range = qi + lane < nq;
-        const uint32_t key_l = in_range ? cv.keys[s0 + lane] : 0u;
-        const uint32_t key0 = lane_u32(key_l, 0);
-        const int cz0 = static_cast<int>(key0 & zmask);
-        const int cz_l = static_cast<int>(key_l & zmask);
-        const bool zok = in_range && abs(cz_l - cz0) <= a.group_z;
-        const uint32_t shift = g.bz + 2u;
-        const uint64_t mm = __ballot(zok && (key_l >> shift) == (key0 >> shift));
-        const int gm = (~mm == 0ull) ? 64 : __builtin_ctzll(~mm);
-        int zl = lane < gm ? cz_l : cz0, zh = zl;
+    const bool valid = lane < nq;
+    const uint64_t s = valid ? cv.qord[q0 + lane] : q0;
+    const double qx = valid ? cv.sx[s] : 0.0;
+    const double qy = valid ? cv.sy[s] : 0.0;
+    const double qz = valid ? cv.sz[s] : 0.0;
+    const float r = a.r;
+    // (beyond 1e18 the faces' FP32 arithmetic could overflow)
+    bool pending = valid && fabs(qx) < 1e18 && fabs(qy) < 1e18 && fabs(qz) < 1e18 && r < 1e18f &&
+                   r > 1e-18f;
+    uint64_t left = __ballot(valid && !pending);  // rows for k_radius_rest
+    for (;;) {
+        const uint64_t pm = __ballot(pending);
+        if (!pm) break;
+        const int first = __builtin_ctzll(pm);
+        const double bx = lane_value(qx, first), by = lane_value(qy, first),
+                     bz = lane_value(qz, first);
+        const float rx = static_cast<float>(qx - bx), ry = static_cast<float>(qy - by),
+                    rz = static_cast<float>(qz - bz);
+        bool act = pending;
+        bool got = false;
+        StageBox B;
+        for (;;) {
+            const float lx = wave_min_f32(act ? rx : INFINITY), ux = -wave_min_f32(act ? -rx : INFINITY);
+            const float ly = wave_min_f32(act ? ry : INFINITY), uy = -wave_min_f32(act ? -ry : INFINITY);
+            const float lz = wave_min_f32(act ? rz : INFINITY), uz = -wave_min_f32(act ? -rz : INFINITY);
+            // Faces at least r from every active query: the offsets' FP32
+            // rounding and the FP64 rounding of the faces taken off.
+            const float W = fmaxf(fmaxf(fmaxf(-lx, ux), fmaxf(-ly, uy)), fmaxf(-lz, uz)) + r;
+            const double pad = static_cast<double>(r) + 3e-7 * static_cast<double>(W) + a.margin;
+            B.X0 = bx + static_cast<double>(lx) - pad;
+            B.X1 = bx + static_cast<double>(ux) + pad;
+            B.Y0 = by + static_cast<double>(ly) - pad;
+            B.Y1 = by + static_cast<double>(uy) + pad;
+            B.Z0 = bz + static_cast<double>(lz) - pad;
+            B.Z1 = bz + static_cast<double>(uz) + pad;
+            // Grid cells by the points' own rule, so that a point inside the
+            // faces is inside the cells.
+            const Box b{uniform_i32(static_cast<int>(cell_coord(B.X0, g.ox, g.inv_c, g.gx))),
+                        uniform_i32(static_cast<int>(cell_coord(B.X1, g.ox, g.inv_c, g.gx))),
+                        uniform_i32(static_cast<int>(cell_coord(B.Y0, g.oy, g.inv_c, g.gy))),
+                        uniform_i32(static_cast<int>(cell_coord(B.Y1, g.oy, g.inv_c, g.gy))),
+                        uniform_i32(static_cast<int>(cell_coord(B.Z0, g.oz, g.inv_cz, g.gz))),
+                        uniform_i32(static_cast<int>(cell_coord(B.Z1, g.oz, g.inv_cz, g.gz)))};
+            const uint64_t ncb = static_cast<uint64_t>(b.x1 - b.x0 + 1) *
+                                 static_cast<uint64_t>(b.y1 - b.y0 + 1);
+            if (ncb <= kStageCols * 64u) {
+                uint32_t lo[kStageCols], len[kStageCols], part = 0;
+                box_columns(ka, wg, b, static_cast<int>(ncb), lane, lo, len);
 #pragma unroll
-        for (int m = 32; m > 0; m >>= 1) {
-            zl = min(zl, __shfl_xor(zl, m));
-            zh = max(zh, __shfl_xor(zh, m));
-        }
-        const double fx = cv.sx[s0], fy = cv.sy[s0];
-        const int qcx = static_cast<int>(cell_coord(fx, g.ox, g.inv_c, g.gx));
-        const int qcy = static_cast<int>(cell_coord(fy, g.oy, g.inv_c, g.gy));
-        const int bx0 = qcx & ~1, by0 = qcy & ~1;
-        const Box box{bx0 - a.rx, bx0 + 1 + a.rx, by0 - a.rx, by0 + 1 + a.rx, zl - a.rz, zh + a.rz};
-        const int ncb = (2 + 2 * a.rx) * (2 + 2 * a.rx);
-        uint32_t tot = 0;
-        for (int cb = 0; cb < ncb; cb += kWave) {
-            uint32_t lo, len;
-            box_ranges(ka, wg, box, cb, lane, 0u, lo, len);
-            tot += lane_u32(wave_incl_scan_u32(len, lane), 63);
-        }
-        const bool cached = ncb <= kWave && tot <= kRadCand;
-        double px[kRadBatches], py[kRadBatches], pz[kRadBatches];
-        uint32_t pj[kRadBatches];
-        uint32_t lo0 = 0, excl0 = 0;
-        if (cached) {
-            uint32_t len;
-            box_ranges(ka, wg, box, 0, lane, 0u, lo0, len);
-            excl0 = wave_incl_scan_u32(len, lane) - len;
-#pragma unroll
-            for (int b = 0; b < kRadBatches; ++b) {
-                px[b] = py[b] = pz[b] = 0.0;
-                pj[b] = kInfU;
-                if (static_cast<uint32_t>(b * 64) < tot) {
-                    const uint32_t t = b * 64 + lane;
-                    const uint32_t j = candidate_pos(lo0, excl0, t);
-                    if (t < tot) {
-                        px[b] = cv.sx[j];
-                        py[b] = cv.sy[j];
-                        pz[b] = cv.sz[j];
-                        pj[b] = j;
+                for (int i = 0; i < kStageCols; ++i) part += min(len[i], 1u << 20);
+                const uint32_t incl = wave_scan_u32(part);
+                const uint32_t N = lane_u32(incl, 63);
+                if (N <= kStageRaw) {
+                    // Cells: as the kNN search's.
+                    const float Lx = static_cast<float>(B.X1 - B.X0), Ly = static_cast<float>(B.Y1 - B.Y0),
+                                Lz = static_cast<float>(B.Z1 - B.Z0);
+                    float cx = r * 0.34f, cy = r * 0.5f, cz = r;
+                    for (;;) {
+                        B.nx = uniform_i32(static_cast<int>(fminf(Lx / cx, 1000.0f)) + 1);
+                        B.ny = uniform_i32(static_cast<int>(fminf(Ly / cy, 1000.0f)) + 1);
+                        B.nz = uniform_i32(Lz > 4.0f * r ? static_cast<int>(fminf(Lz / cz, 1000.0f)) + 1 : 1);
+                        if (static_cast<uint32_t>(B.nx * B.ny * B.nz) <= kStageCells) break;
+                        cx *= 1.3f;
+                        cy *= 1.3f;
+                        cz *= 1.3f;
                     }
+                    B.hx = 1.0f / cx;
+                    B.hy = 1.0f / cy;
+                    B.hz = B.nz > 1 ? 1.0f / cz : 0.0f;
+                    got = stage_points(cv, S, lo, len, incl - part, N, B, lane);
                 }
             }
+            if (got) break;
+            const float dx = ux - lx, dy = uy - ly, dz = uz - lz;
+            const float big = fmaxf(dx, fmaxf(dy, dz));
+            const uint64_t am = __ballot(act);
+            if (!(big > 0.0f) || __popcll(am) <= kRadiusFew) break;
+            // Too many: the half of the group that holds its first query.
+            const float v = dx == big ? rx : (dy == big ? ry : rz);
+            const float mid = 0.5f * (dx == big ? lx + ux : (dy == big ? ly + uy : lz + uz));
+            // (the first query is the base: its offset is 0)
+            const bool keep = act && (v <= mid) == (0.0f <= mid);
+            if (__ballot(keep) == am) break;  // the extent is within rounding
+            act = keep;
         }
-        for (int gi = 0; gi < gm; ++gi) {
-            const uint64_t s = s0 + gi;
-            const double qx = cv.sx[s], qy = cv.sy[s], qz = cv.sz[s];
-            uint32_t cnt = 0;
-            double sx = 0.0, sy = 0.0, sz = 0.0;
-            double c[6] = {0, 0, 0, 0, 0, 0};
-            for (int pass = 0; pass < (a.mode == 0 ? 2 : 1); ++pass) {
-                double mx = 0.0, my = 0.0, mz = 0.0;
-                if (pass == 1) {
-                    const double nn = static_cast<double>(cnt);
-                    mx = wave_sum_f64(sx) / nn;
-                    my = wave_sum_f64(sy) / nn;
-                    mz = wave_sum_f64(sz) / nn;
-                }
-                if (cached) {
-                    if (pass == 0)
-                        radius_pass1(px, py, pz, pj, tot, qx, qy, qz, a.r2, cnt, sx, sy, sz);
-                    else
-                        radius_pass2(px, py, pz, pj, tot, qx, qy, qz, a.r2, mx, my, mz, c);
-                    continue;
-                }
-                // Streamed: chunks of 64 columns and 256 candidates.
-                for (int cb = 0; cb < ncb; cb += kWave) {
-                    uint32_t lo, len;
-                    box_ranges(ka, wg, box, cb, lane, 0u, lo, len);
-                    const uint32_t incl = wave_incl_scan_u32(len, lane);
-                    const uint32_t ctot = lane_u32(incl, 63);
-                    const uint32_t excl = incl - len;
-                    for (uint32_t t0 = 0; t0 < ctot; t0 += kRadCand) {
-                        double cx[kRadBatches], cy[kRadBatches], czv[kRadBatches];
-                        uint32_t cj[kRadBatches];
-                        const uint32_t n1 = min(ctot - t0, kRadCand);
+        if (!got) {  // the rest of the wave is as dense
+            left |= __ballot(pending);
+            break;
+        }
+        // The lane's cells: rows and layers [*0, *1], a hair wider than r, so
+        // that rounding loses no point.
+        const float fx = static_cast<float>(qx - B.X0), fy = static_cast<float>(qy - B.Y0),
+                    fz = static_cast<float>(qz - B.Z0);
+        const float e = r * 1.0001f + 1e-6f * (fabsf(fx) + fabsf(fy) + fabsf(fz)) +
+                        static_cast<float>(a.margin);
+        int cx0 = 0, cx1 = 0, cy0 = 0, cy1 = -1, cz0 = 0, cz1 = -1;
+        if (act) {
+            cx0 = min(static_cast<int>(fmaxf(fx - e, 0.0f) * B.hx), B.nx - 1);
+            cx1 = min(static_cast<int>((fx + e) * B.hx), B.nx - 1);
+            cy0 = static_cast<int>(fmaxf(fy - e, 0.0f) * B.hy);
+            cy1 = min(static_cast<int>((fy + e) * B.hy), B.ny - 1);
+            cz0 = min(static_cast<int>(fmaxf(fz - e, 0.0f) * B.hz), B.nz - 1);
+            cz1 = min(static_cast<int>((fz + e) * B.hz), B.nz - 1);
+        }
+        const double r2 = act ? a.r2 : -1.0;
+        auto walk = [&](auto&& take) {
+            for (int dz = 0; __ballot(cz0 + dz <= cz1); ++dz)
+                for (int dy = 0; __ballot(cy0 + dy <= cy1); ++dy) {
+                    uint32_t p = 0, end = 0;
+                    if (cy0 + dy <= cy1 && cz0 + dz <= cz1) {
+                        const int row = ((cz0 + dz) * B.ny + cy0 + dy) * B.nx;
+                        p = S.cell[row + cx0];
+                        end = S.cell[row + cx1 + 1];
+                    }
+                    while (__ballot(p < end)) {
 #pragma unroll
-                        for (int b = 0; b < kRadBatches; ++b) {
-                            cx[b] = cy[b] = czv[b] = 0.0;
-                            cj[b] = kInfU;
-                            if (static_cast<uint32_t>(b * 64) < n1) {
-                                const uint32_t t = t0 + b * 64 + lane;
-                                const uint32_t j = candidate_pos(lo, excl, t);
-                                if (t < ctot) {
-                                    cx[b] = cv.sx[j];
-                                    cy[b] = cv.sy[j];
-                                    czv[b] = cv.sz[j];
-                                    cj[b] = j;
-                                }
-                            }
+                        for (int i = 0; i < 4; ++i) {
+                            const uint32_t t = p < end ? p : 0u;
+                            // (px - qx: the negative of KD3Index's difference,
+                            // with the same square)
+                            const double px = S.x[t] - qx, py = S.y[t] - qy, pz = S.z[t] - qz;
+                            double d2 = px * px;
+                            d2 = d2 + py * py;
+                            d2 = d2 + pz * pz;
+                            take(px, py, pz, p < end && d2 < r2);
+                            ++p;
                         }
-                        if (pass == 0)
-                            radius_pass1(cx, cy, czv, cj, n1, qx, qy, qz, a.r2, cnt, sx, sy, sz);
-                        else
-                            radius_pass2(cx, cy, czv, cj, n1, qx, qy, qz, a.r2, mx, my, mz, c);
                     }
                 }
-            }
-            if (a.mode == 1) {
-                if (lane == 0) a.counts[cv.perm[s]] = cnt;
-                continue;
-            }
-            const double den = static_cast<double>(cnt) - 1.0;
-            double v[6];
-#pragma unroll
-            for (int i = 0; i < 6; ++i) v[i] = wave_sum_f64(c[i]) / den;
-            if (lane == 0) {
-                double* rec = a.cov + kCovRecord * s;
-#pragma unroll
-                for (int i = 0; i < 6; ++i) rec[i] = v[i];
-                reinterpret_cast<uint64_t*>(rec)[6] = 0;
-                reinterpret_cast<uint64_t*>(rec)[7] = cnt;
-            }
+        };
+        uint32_t cnt = 0;
+        double sx = 0.0, sy = 0.0, sz = 0.0;
+        double c[6] = {0, 0, 0, 0, 0, 0};
+        if (a.mode == 1) {
+            walk([&](double, double, double, bool in) { cnt += in ? 1u : 0u; });
+        } else {
+            walk([&](double px, double py, double pz, bool in) {
+                cnt += in ? 1u : 0u;
+                sx += in ? px : 0.0;
+                sy += in ? py : 0.0;
+                sz += in ? pz : 0.0;
+            });
+            const double nn = static_cast<double>(cnt);
+            const double mx = sx / nn, my = sy / nn, mz = sz / nn;
+            walk([&](double px, double py, double pz, bool in) {
+                const double dx = in ? px - mx : 0.0, dy = in ? py - my : 0.0,
+                             dz = in ? pz - mz : 0.0;
+                c[0] += dx * dx;
+                c[1] += dx * dy;
+                c[2] += dx * dz;
+                c[3] += dy * dy;
+                c[4] += dy * dz;
+                c[5] += dz * dz;
+            });
         }
-        qi += gm;
+        if (act) write_radius_row(a, s, cnt, c);
+        pending = pending && !act;
+        wave_lds_order();
     }
+    if (left) {
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(a.rest, static_cast<uint32_t>(__popcll(left)));
+        at = lane_u32(at, 0) + lanes_below64(left);
+        if ((left >> lane) & 1ull) a.rest[1 + at] = static_cast<uint32_t>(s);
+    }
+}
+
+// The rows k_radius left, their number read on the device.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_radius_rest(RadiusArgs a)
+{
+    KnnArgs ka{};
+    ka.cv = a.cv;
+    WaveGrid wg{};
+    wg.g = a.cv.g;
+    wg.colstart = a.cv.colstart;
+    const uint32_t total = a.rest[0];
+    for (uint32_t i = blockIdx.x; i < total; i += gridDim.x)
+        radius_row(a, ka, wg, uniform_u32(a.rest[1 + i]), __lane_id());
 }
 
 // Per sorted row: eigensystem of the stored covariance and every requested
@@ -2353,7 +2516,7 @@ void launch_knn(const CloudView& cv, const FusedProgram& prog, int mode,
 }
 
 void launch_radius(const CloudView& cv, double radius, int mode, double* cov, uint32_t* counts,
-                   int group_z, hipStream_t s)
+                   uint32_t* rest, hipStream_t s)
 {
     if (cv.n == 0) return;
     RadiusArgs a{};
@@ -2368,12 +2531,16 @@ void launch_radius(const CloudView& cv, double radius, int mode, double* cov, ui
     const double slack = 1e-15 * (span + fabs(g.ox) + fabs(g.oy) + fabs(g.oz));
     a.rx = static_cast<int32_t>(ceil((radius + slack) / g.c));
     a.rz = static_cast<int32_t>(ceil((radius + slack) / g.cz));
-    a.group_z = group_z;
+    a.r = nextafterf(static_cast<float>(radius), INFINITY);
+    a.margin = 1e-6 * fmin(g.c, g.cz) + slack + 1e-300;
     a.mode = mode;
     a.cov = cov;
     a.counts = counts;
-    const uint32_t blocks = div_up(cv.n, 256);
-    hipLaunchKernelGGL(k_radius, dim3(blocks), dim3(256), 0, s, a);
+    a.rest = rest;
+    launch_fill_u32(rest, 1, 0u, s);
+    hipLaunchKernelGGL(k_radius, dim3(div_up(cv.n, 64)), dim3(64), 0, s, a);
+    const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>(cv.n, 8192));
+    hipLaunchKernelGGL(k_radius_rest, dim3(blocks), dim3(64), 0, s, a);
 }
 
 void launch_features(const CloudView& cv, const FusedProgram& prog,

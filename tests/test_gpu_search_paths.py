@@ -11,6 +11,15 @@ from helpers import set_equal_rows, small_cloud
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture
+def ctx():
+    # One of this test's own: the flags of re-solved rows follow the grid, and
+    # a shared context may hold autotuned grids.
+    c = g.Context(0)
+    yield c
+    c.close()
+
+
 def cloud(kind):
     rng = np.random.default_rng(81)
     if kind == "ragged":  # last wave of one query
@@ -79,3 +88,32 @@ def test_batch_instances_agree(knns):
                                   np.asarray(b.tile(cb, t)).view(np.uint64)), (t, k)
     b.close()
     c.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 4097])
+@pytest.mark.parametrize("per", [4, 40, 250, 450, 900])
+def test_radius_paths_agree(ctx, oracle, n, per):
+    # From a few neighbors (whole groups staged) over halved groups to rows
+    # streamed one by one, and waves with both.  Counts are exact; moments of
+    # up to n points of size r differ from numpy's by n eps r^2.
+    rng = np.random.default_rng(84)
+    p = np.column_stack([rng.uniform(0, 40.0, (n, 2)), rng.uniform(0, 0.4, n)])
+    p[n // 2:, :2] *= 0.25
+    r = float(np.sqrt(per * 1600.0 / (np.pi * n)))
+    x, y, z = np.ascontiguousarray(p.T)
+    cl = ctx.cloud(x, y, z)
+    want = oracle.kd3(x, y, z).radius_counts(r)
+    assert np.array_equal(cl.radius_counts(r), want)
+    (cols,), (status,) = cl.run([g.stage(g.STAGE_EIGENVALUES, 8, radius=r, min_k=3)],
+                                init=np.nan)
+    cl.close()
+    rows = np.flatnonzero(want >= 3)[::37]
+    got = np.array([c[rows] for c in cols]).T
+    d = p[rows][:, None, :] - p[None]
+    near = np.einsum("ijk,ijk->ij", d, d) < r * r
+    for i, m in zip(range(len(rows)), near):
+        if m.sum() != want[rows[i]]:
+            continue  # a distance that rounds to r otherwise than KD3Index's
+        ev = np.linalg.eigvalsh(np.cov(p[m].T))
+        tol = 64 * m.sum() * np.finfo(np.float64).eps * max(r * r, ev[-1])
+        assert np.all(np.abs(got[i] - ev) <= tol), (n, per, rows[i])
