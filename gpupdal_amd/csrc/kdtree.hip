@@ -55,11 +55,12 @@ __device__ __forceinline__ const double* axis(const KdView& t, int f)
 }
 
 // ------------------------------------------------------------- building --
-// Two regimes.  Nodes of more than kSub points ("big") are split level by
+// Three regimes.  Nodes of more than kMid points ("big") are split level by
 // level over the whole device: every kernel of a level walks only the points
 // of the level's big nodes (an "active index" t maps to a node by binary
-// search over the nodes' point-count prefix, then to its position).  A node
-// of at most kSub points ("small") is handed to one workgroup, which loads
+// search over the nodes' point-count prefix, then to its position).  Smaller
+// nodes are split by one workgroup each (k_kd_middle).  A node of at most the
+// subtree size (<= kSub points) ("small") is handed to one workgroup, which loads
 // its points into LDS and builds its whole subtree there, level by level
 // with block barriers.
 constexpr uint32_t kSub = 4096;           // small-node capacity (points)
@@ -867,6 +868,202 @@ __global__ __launch_bounds__(kLvlThreads) void k_kd_big_minmax(
                 atomicMax(&t.mx[3 * nd + d], s_hi[j * 3 + d]);
             }
         }
+    }
+}
+
+// -------------------------------------------------------- middle nodes --
+// Nodes of more points than a subtree workgroup holds but at most kMid: one
+// workgroup each splits them, depth first, until every part fits a subtree
+// workgroup.  A pass over a node keeps the predicate as one bit per point in
+// LDS (a word per 64 points, with the words' prefix counts), so the ranks and
+// partners of the Hoare pairing need no further pass over the coordinates.
+// The midpoint cuts of uneven clouds leave long chains of such nodes; as
+// device-wide levels each costs ten launches however few its points (4M
+// points: 24 levels; 250k: 20).
+//
+// Bound by the latency of the passes over one node.  With every node above the
+// subtree size (2048) split by device-wide levels the runs that wait for the
+// tree took, ms: 48k points 1.88, 250k 2.18, 4M 8.7; with this 1.70, 1.57, 8.2.
+// kMid: a word of predicate bits per thread; twice it would need two, and
+// leaves 250k points only eight workgroups.
+constexpr uint32_t kMid = 16384;
+constexpr int kMidThreads = 256;  // a word per thread covers kMid points
+constexpr uint32_t kMidParts = 16;  // kMid or 16 parts of the subtree size, the smaller
+
+struct MidFrame {
+    double box[6];
+    uint32_t nd, lo, hi;
+};
+
+struct MidShared {
+    unsigned long long mask[kMidThreads];
+    uint32_t pre[kMidThreads];
+    uint16_t partner[kMid / 2];
+    unsigned long long mn[3], mx[3];
+    MidFrame frames[kMidParts + 2];
+    int depth;
+    uint32_t own;   // the workgroup's list slot is taken
+};
+
+// One Hoare pass over [s, e): the points with coordinate < cut (<= cut) first.
+// Returns their number.
+template <bool kEqual>
+__device__ __forceinline__ uint32_t mid_pass(const KdView& t, MidShared& S, const double* ax,
+                                             double cv, uint32_t s, uint32_t e)
+{
+    const uint32_t tid = threadIdx.x;
+    const int lane = __lane_id();
+    const uint32_t len = e - s, groups = (len + 63u) >> 6;
+#pragma unroll 4
+    for (uint32_t g = tid >> 6; g < groups; g += kMidThreads / 64) {
+        const uint32_t i = g * 64u + lane;
+        const double v = i < len ? ax[s + i] : 0.0;
+        const unsigned long long m = __ballot(i < len && (kEqual ? v <= cv : v < cv));
+        if (lane == 0) S.mask[g] = m;
+    }
+    __syncthreads();
+    uint32_t L;
+    const uint32_t before = kd_block_scan<kMidThreads>(
+        tid < groups ? static_cast<uint32_t>(__popcll(S.mask[tid])) : 0u, &L);
+    if (tid < groups) S.pre[tid] = before;
+    __syncthreads();
+    if (L == 0 || L == len) return L;  // nothing misplaced
+    // Misplaced on the right, by their rank from the right.
+    for (uint32_t i = L + tid; i < len; i += kMidThreads) {
+        const unsigned long long m = S.mask[i >> 6];
+        if (!((m >> (i & 63u)) & 1ull)) continue;
+        const uint32_t below = S.pre[i >> 6] +
+                               static_cast<uint32_t>(__popcll(m & ((1ull << (i & 63u)) - 1ull)));
+        S.partner[L - 1u - below] = static_cast<uint16_t>(i);
+    }
+    __syncthreads();
+    // Misplaced on the left, by their rank from the left.
+    for (uint32_t i = tid; i < L; i += kMidThreads) {
+        const unsigned long long m = S.mask[i >> 6];
+        if ((m >> (i & 63u)) & 1ull) continue;
+        const uint32_t below = S.pre[i >> 6] +
+                               static_cast<uint32_t>(__popcll(m & ((1ull << (i & 63u)) - 1ull)));
+        const uint32_t p = s + i, q = s + S.partner[i - below];
+        const uint32_t vp = t.vind[p], vq = t.vind[q];
+        const double xp = t.px[p], yp = t.py[p], zp = t.pz[p];
+        const double xq = t.px[q], yq = t.py[q], zq = t.pz[q];
+        t.vind[p] = vq;
+        t.px[p] = xq;
+        t.py[p] = yq;
+        t.pz[p] = zq;
+        t.vind[q] = vp;
+        t.px[q] = xp;
+        t.py[q] = yp;
+        t.pz[q] = zp;
+    }
+    __syncthreads();
+    return L;
+}
+
+__global__ __launch_bounds__(kMidThreads) void k_kd_middle(KdView t, uint32_t* __restrict__ small,
+                                                           uint32_t list_cap,
+                                                           uint32_t* __restrict__ hdr, uint32_t sub)
+{
+    __shared__ MidShared S;
+    const uint32_t tid = threadIdx.x;
+    const int lane = __lane_id();
+    const uint32_t nd0 = small[blockIdx.x];
+    if (t.nr[nd0] - t.nl[nd0] <= sub) return;
+    if (tid == 0) {
+        S.depth = 1;
+        S.own = 0;
+        S.frames[0].nd = nd0;
+        S.frames[0].lo = t.nl[nd0];
+        S.frames[0].hi = t.nr[nd0];
+        for (int i = 0; i < 6; ++i) S.frames[0].box[i] = t.box[6 * static_cast<size_t>(nd0) + i];
+    }
+    __syncthreads();
+    for (;;) {
+        const int depth = S.depth;
+        if (depth == 0) break;
+        const double* box = S.frames[depth - 1].box;
+        const uint32_t nd = S.frames[depth - 1].nd;
+        const uint32_t first = S.frames[depth - 1].lo, last = S.frames[depth - 1].hi;
+        __syncthreads();
+        if (tid < 3) {
+            S.mn[tid] = ~0ull;
+            S.mx[tid] = 0ull;
+        }
+        unsigned long long lo[3] = {~0ull, ~0ull, ~0ull}, hi[3] = {0ull, 0ull, 0ull};
+#pragma unroll 4
+        for (uint32_t p = first + tid; p < last; p += kMidThreads) {
+            const unsigned long long v[3] = {enc_order(t.px[p]), enc_order(t.py[p]),
+                                             enc_order(t.pz[p])};
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                lo[d] = v[d] < lo[d] ? v[d] : lo[d];
+                hi[d] = v[d] > hi[d] ? v[d] : hi[d];
+            }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const unsigned long long ol = __shfl_xor(lo[d], o), oh = __shfl_xor(hi[d], o);
+                lo[d] = ol < lo[d] ? ol : lo[d];
+                hi[d] = oh > hi[d] ? oh : hi[d];
+            }
+        __syncthreads();
+        if (lane == 0)
+            for (int d = 0; d < 3; ++d) {
+                atomicMin(&S.mn[d], lo[d]);
+                atomicMax(&S.mx[d], hi[d]);
+            }
+        __syncthreads();
+        double mn[3], mx[3];
+        for (int d = 0; d < 3; ++d) {
+            mn[d] = dec_order(S.mn[d]);
+            mx[d] = dec_order(S.mx[d]);
+        }
+        int f;
+        double cv;
+        kd_choose_split(box, mn, mx, f, cv);
+        const uint32_t lim1 = mid_pass<false>(t, S, axis(t, f), cv, first, last);
+        const uint32_t lim2 = lim1 + mid_pass<true>(t, S, axis(t, f), cv, first + lim1, last);
+        if (tid == 0) {
+            kd_parent_div(t, nd, mn, mx);
+            t.feat[nd] = f;
+            t.cutval[nd] = cv;
+            double b[6];  // (the frame is written over below)
+            for (int i = 0; i < 6; ++i) b[i] = box[i];
+            const uint32_t cnt = last - first;
+            const uint32_t idx = kd_split_index(cnt, lim1, lim2);
+            const uint32_t c1 = atomicAdd(&hdr[kHdrNodes], 2u);
+            int top = depth - 1;
+            if (c1 + 1 >= t.cap) {
+                hdr[kHdrOverflow] = kOvfNodes;  // the build is redone
+                top = 0;
+            } else {
+                kd_make_children(t, nd, first, idx, last, c1, f, cv, b);
+                for (int c = 0; c < 2; ++c) {
+                    const uint32_t cl = c ? first + idx : first, ch = c ? last : first + idx;
+                    if (ch - cl > sub) {
+                        MidFrame& n = S.frames[top++];
+                        n.nd = c1 + c;
+                        n.lo = cl;
+                        n.hi = ch;
+                        for (int i = 0; i < 6; ++i) n.box[i] = i == (c ? f : 3 + f) ? cv : b[i];
+                        continue;
+                    }
+                    const uint32_t at = S.own ? atomicAdd(&hdr[kHdrSmall], 1u) : blockIdx.x;
+                    S.own = 1;
+                    if (at < list_cap) {
+                        small[at] = c1 + c;
+                    } else {
+                        hdr[kHdrOverflow] = kOvfLists;
+                        top = 0;
+                        break;
+                    }
+                }
+            }
+            S.depth = top;
+        }
+        __syncthreads();
     }
 }
 
@@ -2075,25 +2272,39 @@ uint32_t launch_kd_build(const double* x, const double* y, const double* z, uint
 {
     const uint32_t sub = std::min<uint32_t>(std::max<uint32_t>(kt.subtree_points, kLeafMax + 1),
                                             kt.small_blocks ? kSubSmall : kSub);
+    const uint32_t mid = std::min(kMid, kMidParts * sub);
     hipLaunchKernelGGL(k_kd_init, dim3(div_up(n, kKdThreads)), dim3(kKdThreads), 0, s, x, y, z,
                        static_cast<uint32_t>(n), t);
     launch_fill_u32(w.hdr, kHdrWords, 0u, s);
     hipLaunchKernelGGL(k_kd_roots, dim3(1), dim3(kChildThreads), 0, s, t, starts, ntiles,
-                       bounds, w, sub);
+                       bounds, w, mid);
     uint32_t h[kHdrWords];
-    GF_HIP(hipMemcpyAsync(h, w.hdr, sizeof(h), hipMemcpyDeviceToHost, s));
-    GF_HIP(hipStreamSynchronize(s));
-    if (h[kHdrOverflow]) return h[kHdrOverflow];
-    uint32_t A = h[kHdrA], P = h[kHdrP], nsmall = h[kHdrSmall];
+    auto read_header = [&] {
+        GF_HIP(hipMemcpyAsync(h, w.hdr, sizeof(h), hipMemcpyDeviceToHost, s));
+        GF_HIP(hipStreamSynchronize(s));
+        return h[kHdrOverflow];
+    };
+    uint32_t A, P, nsmall;
+    if (ntiles == 1) {  // one root, in a list that holds it
+        A = n > mid ? 1u : 0u;
+        P = A ? static_cast<uint32_t>(n) : 0u;
+        nsmall = 1u - A;
+    } else {
+        if (const uint32_t o = read_header()) return o;
+        A = h[kHdrA];
+        P = h[kHdrP];
+        nsmall = h[kHdrSmall];
+    }
     int cur = 0;
-    // Levels are queued kLevelsPerRead at a time; each kernel reads its
-    // level's (A, P) from the header.  Grids are sized from bounds known on
-    // the host: P never grows from one level to the next, A at most doubles.
-    constexpr int kLevelsPerRead = 4;
+    // Levels are queued several at a time (those that halving the nodes
+    // needs, and one more); each kernel reads its level's (A, P) from the
+    // header.  Grids are sized for a bound known on the host: P never grows
+    // from one level to the next.
     while (A) {
-        uint64_t Ab = A;
         const uint32_t Pb = P;
-        for (int l = 0; l < kLevelsPerRead; ++l) {
+        int levels = 2;
+        while (levels < 6 && (P / A) >> (levels - 1) > mid) ++levels;
+        for (int l = 0; l < levels; ++l) {
             const uint32_t* lvl = w.hdr + kHdrLvl + 2 * cur;
             // Pass 1's reduction chooses the level's splits (no split
             // launch); levels of at most kRawSumBlocks blocks skip the scan
@@ -2113,20 +2324,24 @@ uint32_t launch_kd_build(const double* x, const double* y, const double* z, uint
                                    s, t, pass, w.act[cur], w.off[cur], lvl, w.s1, sc, w.tmp);
             }
             hipLaunchKernelGGL(k_kd_big_children, dim3(1), dim3(kChildThreads), 0, s, t,
-                               w.act[cur], w.off[cur], w.s1, w.s2, w, cur ^ 1, sub);
+                               w.act[cur], w.off[cur], w.s1, w.s2, w, cur ^ 1, mid);
             hipLaunchKernelGGL(
                 k_kd_big_minmax,
                 dim3(std::min<uint32_t>(div_up(Pb, kMinMaxChunk), 4096)),
                 dim3(kLvlThreads), 0, s, t, w.act[cur], w.off[cur], lvl, w.hdr, w.act[cur ^ 1],
                 kt.minmax_lds_nodes);
             cur ^= 1;
-            Ab *= 2;
         }
-        GF_HIP(hipMemcpyAsync(h, w.hdr, sizeof(h), hipMemcpyDeviceToHost, s));
-        GF_HIP(hipStreamSynchronize(s));
-        if (h[kHdrOverflow]) return h[kHdrOverflow];
+        if (const uint32_t o = read_header()) return o;
         A = h[kHdrLvl + 2 * cur];
         P = h[kHdrLvl + 2 * cur + 1];
+        nsmall = h[kHdrSmall];
+    }
+    // (one tree that fits a subtree workgroup has no middle node)
+    if (nsmall && (ntiles > 1 || n > sub)) {
+        hipLaunchKernelGGL(k_kd_middle, dim3(nsmall), dim3(kMidThreads), 0, s, t, w.small,
+                           w.list_cap, w.hdr, sub);
+        if (const uint32_t o = read_header()) return o;
         nsmall = h[kHdrSmall];
     }
     if (nsmall) {
@@ -2146,9 +2361,7 @@ uint32_t launch_kd_build(const double* x, const double* y, const double* z, uint
                                dim3(kSubThreads), 0, s, t, w.small, w.hdr, wave_node);
         GF_HIP(hipGetLastError());
     }
-    GF_HIP(hipMemcpyAsync(h, w.hdr, sizeof(h), hipMemcpyDeviceToHost, s));
-    GF_HIP(hipStreamSynchronize(s));
-    if (h[kHdrOverflow]) return h[kHdrOverflow];
+    if (const uint32_t o = read_header()) return o;
     // Subtree reservations may run past the capacity without using those ids.
     *nodes = std::min<uint32_t>(h[kHdrNodes], t.cap);
     return 0;
