@@ -883,11 +883,12 @@ __global__ __launch_bounds__(kLvlThreads) void k_kd_big_minmax(
 //
 // Bound by the latency of the passes over one node.  With every node above the
 // subtree size (2048) split by device-wide levels the runs that wait for the
-// tree took, ms: 48k points 1.88, 250k 2.18, 4M 8.7; with this 1.70, 1.57, 8.2.
-// kMid: a word of predicate bits per thread; twice it would need two, and
-// leaves 250k points only eight workgroups.
-constexpr uint32_t kMid = 16384;
-constexpr int kMidThreads = 256;  // a word per thread covers kMid points
+// tree took, ms: 48k points 1.88, 250k 2.18, 4M 8.7; with this 1.62, 1.56, 7.7.
+// kMid and threads (250k / 4M points, ms): 8192 and 256 2.08 / 8.2 (more
+// levels), 16384 and 256 1.58 / 8.0, and 1024 1.48 / 8.3 (workgroups wait for
+// the search's to drain), 32768 and 512 1.56 / 7.7.
+constexpr uint32_t kMid = 32768;
+constexpr int kMidThreads = 512;  // a word per thread covers kMid points
 constexpr uint32_t kMidParts = 16;  // kMid or 16 parts of the subtree size, the smaller
 
 struct MidFrame {

@@ -25,8 +25,8 @@ def cloud(kind, n):
 
 
 @pytest.mark.parametrize("kind", ["even", "chain", "lattice", "point"])
-@pytest.mark.parametrize("n,sub", [(2048, 2048), (2049, 2048), (4097, 4096), (16384, 2048),
-                                   (16385, 2048), (40000, 2048), (1700, 101), (1616, 101),
+@pytest.mark.parametrize("n,sub", [(2048, 2048), (2049, 2048), (4097, 4096), (32768, 2048),
+                                   (32769, 2048), (70000, 2048), (1700, 101), (1616, 101),
                                    (9000, 512)])
 def test_middle_nodes_equal_kd3(kind, n, sub):
     x, y, z = cloud(kind, n)
