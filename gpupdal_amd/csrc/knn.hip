@@ -1422,7 +1422,7 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
                     const int row = ((cz0 + dz) * B.ny + cy0 + dy) * B.nx;
                     p = S.cell[row + cx0] + part;
                     e = S.cell[row + cx1 + 1];
-                    seen += e - p;
+                    seen += p < e ? (e - p + LPQ - 1) / LPQ : 0u;
                 }
                 while (__ballot(p < e)) {
 #pragma unroll
