@@ -28,6 +28,7 @@
 #include "gf_eigen.hpp"
 #include "gf_internal.hpp"
 #include "gf_kernels.hpp"
+#include "gf_stage.hpp"
 #include "gf_wave.hpp"
 
 namespace gf {
@@ -1010,13 +1011,6 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_wave_barrier();
 }
 
-// A box staged in LDS: its faces and its cells (counts and 1 / edges).
-struct StageBox {
-    double X0 = 0, X1 = 0, Y0 = 0, Y1 = 0, Z0 = 0, Z1 = 0;
-    float hx = 0, hy = 0, hz = 0;
-    int nx = 1, ny = 1, nz = 1;
-};
-
 // Stages the points of N <= kStageRaw column entries (lo, len: the lane's
 // columns; at: entries of the lanes before it) that lie inside B's faces,
 // counting-sorted by cell.  False if there are more than kStageMax.
@@ -1374,31 +1368,22 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
             pending = pending && !act;
             continue;
         }
-        // The lane's cells at radius rl: rows and layers [*0, *1].
+        // The lane's cells at radius rl.
         float rl = r;
-        int cx0 = 0, cx1 = 0, cy0 = 0, cy1 = -1, cz0 = 0, cz1 = 0;
         const float fx = static_cast<float>(qx - B.X0), fy = static_cast<float>(qy - B.Y0),
                     fz = static_cast<float>(qz - B.Z0);
-        auto cells = [&](float rr) {
-            // A hair wider than rr, so that rounding loses no point.
-            const float e = rr * 1.0001f + 1e-6f * (fabsf(fx) + fabsf(fy) + fabsf(fz)) +
+        // (a hair wider than the radius, so that rounding loses no point)
+        const float wider = 1e-6f * (fabsf(fx) + fabsf(fy) + fabsf(fz)) +
                             static_cast<float>(wg.margin);
-            cx0 = min(static_cast<int>(fmaxf(fx - e, 0.0f) * B.hx), B.nx - 1);
-            cx1 = min(static_cast<int>((fx + e) * B.hx), B.nx - 1);
-            cy0 = static_cast<int>(fmaxf(fy - e, 0.0f) * B.hy);
-            cy1 = act ? min(static_cast<int>((fy + e) * B.hy), B.ny - 1) : cy0 - 1;
-            cz0 = min(static_cast<int>(fmaxf(fz - e, 0.0f) * B.hz), B.nz - 1);
-            cz1 = act ? min(static_cast<int>((fz + e) * B.hz), B.nz - 1) : cz0 - 1;
-        };
-        cells(r);
+        CellRange w = stage_range(B, act, fx, fy, fz, r * 1.0001f + wider);
         // Where the box is denser around this query than its radius asks for,
         // a smaller one.
         {
             uint32_t seen = 0;
-            for (int z = cz0; z <= cz1; ++z)
-                for (int y = cy0; y <= cy1; ++y) {
+            for (int z = w.z0; z <= w.z1; ++z)
+                for (int y = w.y0; y <= w.y1; ++y) {
                     const int row = (z * B.ny + y) * B.nx;
-                    seen += S.cell[row + cx1 + 1] - S.cell[row + cx0];
+                    seen += S.cell[row + w.x1 + 1] - S.cell[row + w.x0];
                 }
             // At least a quarter of those seen are inside the radius, and
             // their number falls at most with its cube.
@@ -1406,7 +1391,7 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
             const float want = kListFactor * static_cast<float>(fetch + 1);
             if (in > want) {
                 rl = fminf(fmaxf(r * cbrtf(want / in), r_need), r);
-                cells(rl);
+                w = stage_range(B, act, fx, fy, fz, rl * 1.0001f + wider);
             }
         }
         cnt_pass += static_cast<uint64_t>(__popcll(__ballot(act)));
@@ -1415,13 +1400,13 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
         double E = act ? E0 : -1.0;
         uint32_t cnt = 0, seen = 0;
         bool cut = false;   // entries below E0 may have been left out
-        for (int dz = 0; __ballot(cz0 + dz <= cz1); ++dz) {
-            for (int dy = 0; __ballot(cy0 + dy <= cy1); ++dy) {
+        for (int dz = 0; __ballot(w.z0 + dz <= w.z1); ++dz) {
+            for (int dy = 0; __ballot(w.y0 + dy <= w.y1); ++dy) {
                 uint32_t p = 0, e = 0;
-                if (cy0 + dy <= cy1 && cz0 + dz <= cz1) {
-                    const int row = ((cz0 + dz) * B.ny + cy0 + dy) * B.nx;
-                    p = S.cell[row + cx0] + part;
-                    e = S.cell[row + cx1 + 1];
+                if (w.y0 + dy <= w.y1 && w.z0 + dz <= w.z1) {
+                    const int row = ((w.z0 + dz) * B.ny + w.y0 + dy) * B.nx;
+                    p = S.cell[row + w.x0] + part;
+                    e = S.cell[row + w.x1 + 1];
                     seen += p < e ? (e - p + LPQ - 1) / LPQ : 0u;
                 }
                 while (__ballot(p < e)) {
@@ -2242,30 +2227,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             left |= __ballot(pending);
             break;
         }
-        // The lane's cells: rows and layers [*0, *1], a hair wider than r, so
-        // that rounding loses no point.
+        // The lane's cells, a hair wider than r, so that rounding loses no
+        // point.
         const float fx = static_cast<float>(qx - B.X0), fy = static_cast<float>(qy - B.Y0),
                     fz = static_cast<float>(qz - B.Z0);
         const float e = r * 1.0001f + 1e-6f * (fabsf(fx) + fabsf(fy) + fabsf(fz)) +
                         static_cast<float>(a.margin);
-        int cx0 = 0, cx1 = 0, cy0 = 0, cy1 = -1, cz0 = 0, cz1 = -1;
-        if (act) {
-            cx0 = min(static_cast<int>(fmaxf(fx - e, 0.0f) * B.hx), B.nx - 1);
-            cx1 = min(static_cast<int>((fx + e) * B.hx), B.nx - 1);
-            cy0 = static_cast<int>(fmaxf(fy - e, 0.0f) * B.hy);
-            cy1 = min(static_cast<int>((fy + e) * B.hy), B.ny - 1);
-            cz0 = min(static_cast<int>(fmaxf(fz - e, 0.0f) * B.hz), B.nz - 1);
-            cz1 = min(static_cast<int>((fz + e) * B.hz), B.nz - 1);
-        }
+        const CellRange w = stage_range(B, act, fx, fy, fz, e);
         const double r2 = act ? a.r2 : -1.0;
         auto walk = [&](auto&& take) {
-            for (int dz = 0; __ballot(cz0 + dz <= cz1); ++dz)
-                for (int dy = 0; __ballot(cy0 + dy <= cy1); ++dy) {
+            for (int dz = 0; __ballot(w.z0 + dz <= w.z1); ++dz)
+                for (int dy = 0; __ballot(w.y0 + dy <= w.y1); ++dy) {
                     uint32_t p = 0, end = 0;
-                    if (cy0 + dy <= cy1 && cz0 + dz <= cz1) {
-                        const int row = ((cz0 + dz) * B.ny + cy0 + dy) * B.nx;
-                        p = S.cell[row + cx0];
-                        end = S.cell[row + cx1 + 1];
+                    if (w.y0 + dy <= w.y1 && w.z0 + dz <= w.z1) {
+                        const int row = ((w.z0 + dz) * B.ny + w.y0 + dy) * B.nx;
+                        p = S.cell[row + w.x0];
+                        end = S.cell[row + w.x1 + 1];
                     }
                     while (__ballot(p < end)) {
 #pragma unroll

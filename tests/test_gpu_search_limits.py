@@ -1,0 +1,50 @@
+"""The search at the limits of its staged boxes' arithmetic: clouds whose cells are
+tiny beside their coordinates, at row counts that leave lanes of the last wave
+without a query.  Lists hold the oracle's KD3 neighbors, and feature columns and
+statuses equal the growing search's, bit for bit, for a cloud and a batch."""
+import numpy as np
+import pytest
+
+import gpupdal_amd as g
+from helpers import set_equal_rows
+
+pytestmark = pytest.mark.gpu
+
+
+def cloud(kind, n):
+    rng = np.random.default_rng(n)
+    if kind == "coincident":  # one place, at negative y
+        p = np.tile([1.0, -5.0, 0.0], (n, 1))
+    elif kind == "millimetres":  # a fine scan in geocentric coordinates
+        p = rng.uniform(0, 1, (n, 3)) * [0.02, 0.02, 0.002] + [5e5, -4e6, -3e6]
+    else:  # "corner": all coordinates large and negative
+        p = rng.uniform(0, 1, (n, 3)) * [1e-3, 1e-3, 1e-3] - 6.4e6
+    return np.ascontiguousarray(p.T)
+
+
+def same_bits(a, b):
+    assert np.array_equal(a[1][0], b[1][0])
+    for ca, cb in zip(a[0][0], b[0][0]):
+        assert np.array_equal(np.asarray(ca).view(np.uint64), np.asarray(cb).view(np.uint64))
+
+
+@pytest.mark.parametrize("k", [1, 8, 9, 20, 36, 40])
+@pytest.mark.parametrize("n", [63, 65, 100, 333])
+@pytest.mark.parametrize("kind", ["coincident", "millimetres", "corner"])
+def test_limits(oracle, kind, n, k):
+    x, y, z = cloud(kind, n)
+    c, slow = g.Context(0), g.Context(0)
+    slow.set_tuning("set_select", 0)
+    cl = c.cloud(x, y, z)
+    ids, _ = cl.knn(k)
+    # (the oracle's lists are KD3Index's, so rows of coincident points agree too)
+    assert set_equal_rows(ids, oracle.kd3(x, y, z).neighbors_all(k, threads=4)).all()
+    st = [g.stage(g.STAGE_COVFEAT, k + 2, features=g.F_ALL10)]
+    want = slow.cloud(x, y, z).run(st, init=np.nan)
+    same_bits(cl.run(st, init=np.nan), want)
+    b = c.batch([(x, y, z), (x[:50], y[:50], z[:50])])
+    got = b.run(st, init=np.nan)
+    same_bits(([[b.tile(col, 0) for col in got[0][0]]], [b.tile(got[1][0], 0)]), want)
+    b.close()
+    slow.close()
+    c.close()
