@@ -891,7 +891,7 @@ constexpr uint32_t kStageRaw = kStageSlots * 64;
 constexpr uint32_t kStageCells = 512;
 constexpr int kStageCols = 5;          // columns of a box per lane
 constexpr int kListRow = 65;    // LDS words between list positions of the ordered lists
-constexpr uint32_t kSlotMask = 0x3FFu;  // slot in a key's low bits (kStageMax <= 1024)
+static_assert(kStageMax <= kSlotMask + 1);  // a slot fits a key's low bits
 
 template <int P, int Q, int R, int D, int N>
 __device__ __forceinline__ void sort_step(uint32_t (&k)[N])
@@ -1004,6 +1004,16 @@ template <int CAP> struct StageShared {
         uint32_t pos[kStageRaw];      // while staging: sorted positions of the box's columns
     };
 };
+
+// stage_size for a box that every lane holds.
+__device__ __forceinline__ bool size_box(StageBox& B, float r)
+{
+    const bool ok = stage_size(B, r, kStageCells);
+    B.nx = uniform_i32(B.nx);
+    B.ny = uniform_i32(B.ny);
+    B.nz = uniform_i32(B.nz);
+    return ok;
+}
 
 __device__ __forceinline__ void wave_lds_order()
 {
@@ -1226,9 +1236,9 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
     uint32_t* my = S.list + lane;
     // The growing search's box reaches ring_max whole cells from a query's
     // own cell on every side.
-    const float r_cap = static_cast<float>(
-        (static_cast<double>(a.tune.ring_max) * fmin(g.c, g.cz) - 4.0 * wg.margin) * (1.0 - 1e-6));
-    bool pending = valid && isfinite(qx) && isfinite(qy) && isfinite(qz) && r_cap > 0.0f;
+    const double reach = static_cast<double>(a.tune.ring_max) * fmin(g.c, g.cz);
+    const float r_cap = static_cast<float>((reach - 4.0 * wg.margin) * (1.0 - 1e-6));
+    bool pending = valid && stage_takes(reach, wg.margin) && stage_takes_point(qx, qy, qz);
     bool defer = valid && !pending;
     uint32_t tries = 0;
     float r_need = 0.0f;  // the smallest radius worth trying for this lane
@@ -1328,25 +1338,8 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
                 }
                 over = N > kStageRaw || N == 0;
                 if (!over) {
-                    // Cells: a third of the radius along x (runs are cut
-                    // there), half of it along y, the radius along z when the
-                    // box is tall.
-                    const float Lx = static_cast<float>(B.X1 - B.X0), Ly = static_cast<float>(B.Y1 - B.Y0),
-                                Lz = static_cast<float>(B.Z1 - B.Z0);
-                    float cx = r * 0.34f, cy = r * 0.5f, cz = r;
-                    for (;;) {
-                        B.nx = uniform_i32(static_cast<int>(fminf(Lx / cx, 1000.0f)) + 1);
-                        B.ny = uniform_i32(static_cast<int>(fminf(Ly / cy, 1000.0f)) + 1);
-                        B.nz = uniform_i32(Lz > 4.0f * r ? static_cast<int>(fminf(Lz / cz, 1000.0f)) + 1 : 1);
-                        if (static_cast<uint32_t>(B.nx * B.ny * B.nz) <= kStageCells) break;
-                        cx *= 1.3f;
-                        cy *= 1.3f;
-                        cz *= 1.3f;
-                    }
-                    B.hx = 1.0f / cx;
-                    B.hy = 1.0f / cy;
-                    B.hz = B.nz > 1 ? 1.0f / cz : 0.0f;
-                    over = !stage_points(cv, S, lo, len, incl - part, N, B, lane);
+                    over = !size_box(B, r) ||
+                           !stage_points(cv, S, lo, len, incl - part, N, B, lane);
                 }
             }
             if (!over) {
@@ -1415,7 +1408,7 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
                         const uint32_t t = p < e ? p : 0u;
                         const uint64_t db = dist_bits(qx, qy, qz, S.x[t], S.y[t], S.z[t]);
                         const double d2 = bits_d2(db);
-                        my[cnt * 64] = (__float_as_uint(static_cast<float>(d2)) & ~kSlotMask) | t;
+                        my[cnt * 64] = list_key(d2, t);
                         cnt += (p < e && d2 < E) ? 1u : 0u;
                         p += LPQ;
                     }
@@ -1426,9 +1419,7 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
 #pragma unroll
                         for (int i = 0; i < TM; ++i) my[i * 64] = k[i];
                         if (cnt >= keep) {
-                            // (the key's bucket ends below this)
-                            E = fmin(E, static_cast<double>(__uint_as_float(
-                                            (my[(keep - 1) * 64] | kSlotMask) + 1u)));
+                            E = fmin(E, key_above(my[(keep - 1) * 64]));
                             cnt = keep;
                             cut = true;
                         }
@@ -1469,10 +1460,9 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
             }
         }
         // The largest coarse distance put in exact order: no entry cut away
-        // has a smaller one (the float rounds a double by 6e-8).
+        // has a smaller one.
         cut = cut || cnt >= keep;
-        const double last = static_cast<double>(__uint_as_float(my[(keep - 1) * 64] & ~kSlotMask)) *
-                            (1.0 - 1.2e-7);
+        const double last = key_below(my[(keep - 1) * 64]);
         // Exact (d2, id) order: neighbors out of order change places
         // until none is (the coarse order is right but for near-equal
         // distances).
@@ -2144,9 +2134,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const double qy = valid ? cv.sy[s] : 0.0;
     const double qz = valid ? cv.sz[s] : 0.0;
     const float r = a.r;
-    // (beyond 1e18 the faces' FP32 arithmetic could overflow)
-    bool pending = valid && fabs(qx) < 1e18 && fabs(qy) < 1e18 && fabs(qz) < 1e18 && r < 1e18f &&
-                   r > 1e-18f;
+    bool pending = valid && stage_takes_point(qx, qy, qz) && r < 1e18f && r > 1e-18f;
     uint64_t left = __ballot(valid && !pending);  // rows for k_radius_rest
     for (;;) {
         const uint64_t pm = __ballot(pending);
@@ -2191,23 +2179,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
                 const uint32_t incl = wave_scan_u32(part);
                 const uint32_t N = lane_u32(incl, 63);
                 if (N <= kStageRaw) {
-                    // Cells: as the kNN search's.
-                    const float Lx = static_cast<float>(B.X1 - B.X0), Ly = static_cast<float>(B.Y1 - B.Y0),
-                                Lz = static_cast<float>(B.Z1 - B.Z0);
-                    float cx = r * 0.34f, cy = r * 0.5f, cz = r;
-                    for (;;) {
-                        B.nx = uniform_i32(static_cast<int>(fminf(Lx / cx, 1000.0f)) + 1);
-                        B.ny = uniform_i32(static_cast<int>(fminf(Ly / cy, 1000.0f)) + 1);
-                        B.nz = uniform_i32(Lz > 4.0f * r ? static_cast<int>(fminf(Lz / cz, 1000.0f)) + 1 : 1);
-                        if (static_cast<uint32_t>(B.nx * B.ny * B.nz) <= kStageCells) break;
-                        cx *= 1.3f;
-                        cy *= 1.3f;
-                        cz *= 1.3f;
-                    }
-                    B.hx = 1.0f / cx;
-                    B.hy = 1.0f / cy;
-                    B.hz = B.nz > 1 ? 1.0f / cz : 0.0f;
-                    got = stage_points(cv, S, lo, len, incl - part, N, B, lane);
+                    got = size_box(B, r) &&
+                          stage_points(cv, S, lo, len, incl - part, N, B, lane);
                 }
             }
             if (got) break;

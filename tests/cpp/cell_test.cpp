@@ -91,4 +91,57 @@ TEST(Cells, RangeHoldsEveryPointInReach)
         }
 }
 
+TEST(Cells, SizingEndsForAnyBox)
+{
+    const float inf = INFINITY;
+    for (double L : {0.0, 1e-300, 1e-9, 1.0, 1e18, 1e30, 1e40, 1e300})
+        for (float r : {0.0f, 1e-45f, 1e-18f, 2.4e-10f, 1.0f, 1e18f, 3e38f, inf})
+            for (double flat : {0.0, 1.0}) {
+                StageBox B;
+                B.X0 = B.Y0 = B.Z0 = -L;
+                B.X1 = B.Y1 = L;
+                B.Z1 = flat * L - (1.0 - flat) * L;
+                const bool ok = stage_size(B, r, 512);
+                if (ok) EXPECT_TRUE(B.nx * B.ny * B.nz <= 512 && B.nx > 0 && B.ny > 0 && B.nz > 0);
+                // Where radius and box are of comparable size it succeeds.
+                if (r >= 1e-18f && r <= 1e18f && L < 1e12 * r) EXPECT_TRUE(ok);
+            }
+}
+
+TEST(Keys, OrderIsThatOfTheDistances)
+{
+    // key_above and key_below bound the distances left out after a cut, at
+    // every scale the search takes and below FLT_MIN.
+    std::mt19937_64 rng(9);
+    std::uniform_real_distribution<double> e(-330.0, std::log10(3.3e37)), u(1.0, 1.0 + 1e-3);
+    for (int t = 0; t < 200000; ++t) {
+        const double a = std::pow(10.0, e(rng));
+        const double b = t % 3 ? a * u(rng) : std::pow(10.0, e(rng));
+        const uint32_t ka = list_key(a, 1023u), kb = list_key(b, 0u);
+        EXPECT_TRUE(std::isfinite(key_value(ka & ~kSlotMask)));
+        if (b >= key_above(ka)) EXPECT_TRUE(kb > ka);
+        if (kb >= ka) EXPECT_TRUE(b >= key_below(ka));
+        EXPECT_TRUE(a < key_above(ka) || a <= 0.0);
+    }
+}
+
+TEST(Keys, RowsTakenHaveFiniteDistances)
+{
+    // The largest coordinate difference of a row the search takes: queries a
+    // kStageFar apart on either side of the origin, and the box's growth.
+    const double reach = kStageFar * (1.0 - 1e-9), margin = reach * 0.2499;
+    EXPECT_TRUE(stage_takes(reach, margin));
+    EXPECT_TRUE(stage_takes_point(-kStageFar * (1.0 - 1e-9), 0.0, 0.0));
+    const double d = 2.0 * kStageFar + reach + 3e-7 * 4.0 * kStageFar + margin;
+    EXPECT_TRUE(std::isfinite(static_cast<float>(3.0 * d * d)));
+    // Spacings whose squares leave FP32's range are refused: the first cells
+    // of clouds 1e20 and 1e40 across, and coordinates that far out.
+    EXPECT_TRUE(!stage_takes(8.0 * 3e19, 1e5));
+    EXPECT_TRUE(!stage_takes(8.0 * 3e39, 1e25));
+    EXPECT_TRUE(!stage_takes_point(0.0, 1e18, 0.0));
+    EXPECT_TRUE(!stage_takes_point(0.0, 0.0, -INFINITY));
+    EXPECT_TRUE(!stage_takes_point(NAN, 0.0, 0.0));
+    EXPECT_TRUE(!stage_takes(1.0, 0.25));
+}
+
 int main(int argc, char** argv) { return mini::run_all(argc, argv); }

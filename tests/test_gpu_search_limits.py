@@ -1,7 +1,8 @@
 """The search at the limits of its staged boxes' arithmetic: clouds whose cells are
-tiny beside their coordinates, at row counts that leave lanes of the last wave
-without a query.  Lists hold the oracle's KD3 neighbors, and feature columns and
-statuses equal the growing search's, bit for bit, for a cloud and a batch."""
+tiny beside their coordinates, or whose distances leave FP32's range when
+squared, at row counts that leave lanes of the last wave without a query.  Lists
+hold the oracle's KD3 neighbors, and feature columns and statuses equal the
+growing search's, bit for bit, for a cloud and a batch."""
 import numpy as np
 import pytest
 
@@ -17,6 +18,8 @@ def cloud(kind, n):
         p = np.tile([1.0, -5.0, 0.0], (n, 1))
     elif kind == "millimetres":  # a fine scan in geocentric coordinates
         p = rng.uniform(0, 1, (n, 3)) * [0.02, 0.02, 0.002] + [5e5, -4e6, -3e6]
+    elif kind.startswith("scale"):  # spacings at and beyond the FP32 keys' range
+        p = rng.normal(size=(n, 3)) * float(kind[5:])
     else:  # "corner": all coordinates large and negative
         p = rng.uniform(0, 1, (n, 3)) * [1e-3, 1e-3, 1e-3] - 6.4e6
     return np.ascontiguousarray(p.T)
@@ -30,7 +33,8 @@ def same_bits(a, b):
 
 @pytest.mark.parametrize("k", [1, 8, 9, 20, 36, 40])
 @pytest.mark.parametrize("n", [63, 65, 100, 333])
-@pytest.mark.parametrize("kind", ["coincident", "millimetres", "corner"])
+@pytest.mark.parametrize("kind", ["coincident", "millimetres", "corner", "scale1e17", "scale1e18",
+                                  "scale1e20", "scale1e40", "scale1e-12", "scale1e-21"])
 def test_limits(oracle, kind, n, k):
     x, y, z = cloud(kind, n)
     c, slow = g.Context(0), g.Context(0)

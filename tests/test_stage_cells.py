@@ -9,7 +9,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 BIN = os.path.join(ROOT, "tests", "cpp", "cell_test")
 
 
-@pytest.mark.parametrize("suite", ["Cells"])
+@pytest.mark.parametrize("suite", ["Cells", "Keys"])
 def test_stage_cells(suite):
     if not os.path.exists(BIN):
         subprocess.run(["make", "-s", "-C", os.path.dirname(BIN), BIN], check=True)
