@@ -105,8 +105,9 @@ struct KnnOutputs {
     uint32_t* ids;           // neighbor-list mode: n x k (original order)
     uint32_t* flagged;       // sorted indices of tie/incomplete rows
     uint32_t* nflagged;      // [0] flagged rows, [1] tie rows, [2] incomplete rows,
-                             // [3] rows in deferred, [4] groups in heavy, [7] next heavy
-                             // half group (8 words cleared before a search)
+                             // [3] rows in deferred, [4] groups in heavy, [5] rows of
+                             // deferred drawn, [7] next heavy half group (8 words
+                             // cleared before a search)
     uint32_t* deferred;      // sorted indices the lane-per-query search leaves to the
                              // growing search (up to one per row)
     uint32_t* heavy;         // query groups whose box holds too many points (up to one

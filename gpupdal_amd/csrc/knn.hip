@@ -36,7 +36,7 @@ namespace gf {
 namespace {
 
 constexpr uint32_t kLaneSmall = 8;     // columns of up to this many points are taken whole
-constexpr int kRegBatches = 8;   // candidates of one row in registers, 64 a batch
+constexpr int kRegBatches = 4;   // candidates of one row in registers, 64 a batch
 constexpr uint32_t kRegCand = kRegBatches * 64;
 constexpr int kGroupBatches = 4; // the same for the box a group of rows shares
 constexpr uint32_t kGroupCand = kGroupBatches * 64;
@@ -1874,28 +1874,48 @@ __device__ __forceinline__ int first_ring(const KnnArgs& a, const WaveGrid& wg, 
 
 // The rows the lane-per-query search left (out.deferred, their count read on
 // the device), or every row (tuning "set_select" 0): one wave per row with
-// the growing search, kRestRows rows per wave so that the covariances of
-// several rows share their passes.
-constexpr int kRestRows = 4;
+// the growing search.  A wave draws a few rows at a time until none is left, so
+// that uneven rows spread and the waves at work stay close together in the
+// cloud; it holds the lists of kRestHeld rows before one lane each forms their
+// covariances.
+//
+// Bound by the latency of one row's chain of loads and selections, so by the
+// waves resident: six per SIMD (80 registers) against four (8 batches of
+// candidates instead of 4).  Draws and flagged rows are atomics on one address,
+// some 50 ns each, hence more rows per draw when there are many.  Search times
+// with four waves, rows of fixed strides and covariances after every four, and
+// as it is now, ms: 500k points with strays far off (every row here), k 16, 160
+// and 94; 60 dense balls, k 16, 10.4 and 6.8; 4M points, k 48, 24.3 and 18.4.
+constexpr uint32_t kRestRows = 4;
+constexpr uint32_t kRestRowsMany = 8;
+constexpr uint32_t kRestMany = 131072;
+constexpr int kRestHeld = 16;
+constexpr uint32_t kRestWaves = 8192;
 
 template <bool kTiled>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_knn_rest(KnnArgs a)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_knn_rest(KnnArgs a)
 {
     extern __shared__ uint32_t s_lds[];
     const int lane = __lane_id();
     uint32_t* scratch = s_lds;
     uint32_t* nbr = s_lds + kScratchWords;
-    const uint64_t total = a.all_rows ? a.cv.n : a.out.nflagged[3];
+    const uint32_t total = a.all_rows ? static_cast<uint32_t>(a.cv.n) : a.out.nflagged[3];
+    const uint32_t per = total >= kRestMany ? kRestRowsMany : kRestRows;
+    // Each wave's first rows are its own; the rest are drawn.
+    const uint32_t drawn0 = gridDim.x * per;
+    uint32_t base = blockIdx.x * per;
+    if (base >= total) return;
     uint64_t cnt[3] = {0, 0, 0};  // search passes, candidates, selections
-    uint64_t nrows = 0;
-    for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kRestRows; base < total;
-         base += static_cast<uint64_t>(gridDim.x) * kRestRows) {
-        const int nq = static_cast<int>(total - base < kRestRows ? total - base : kRestRows);
-        uint8_t my_flags = 0;
-        uint64_t my_s = 0;
-        int my_k = 0;
+    // The rows held: row p's list at nbr + p * lds_stride, its position, size
+    // and flags in lane p.
+    int held = 0;
+    uint8_t my_flags = 0;
+    uint32_t my_s = 0;
+    int my_k = 0;
+    for (;;) {
+        const int nq = base >= total ? 0 : static_cast<int>(min(total - base, per));
         for (int p = 0; p < nq; ++p) {
-            const uint64_t s = a.all_rows ? base + p : a.out.deferred[base + p];
+            const uint32_t s = a.all_rows ? base + p : a.out.deferred[base + p];
             WaveGrid wg;
             if (kTiled) {
                 const TileInfo& ti = a.tiles[tile_of(a.starts, a.ntiles, s)];
@@ -1913,31 +1933,42 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
             bool incomplete = false;
             search_single(a, wg, qx, qy, qz, qcx, qcy, qcz, first_ring(a, wg, qcx, qcy, qcz, lane),
                           lane, scratch, best, incomplete, cnt);
-            finish_query(a, wg, best, incomplete, s, p, lane, nbr, my_flags);
-            if (lane == p) {
+            finish_query(a, wg, best, incomplete, s, held + p, lane, nbr, my_flags);
+            if (lane == held + p) {
                 my_s = s;
                 my_k = wg.k;
             }
-            nrows += 1;
         }
-        if (a.mode != 0) continue;
-        // The lists were written by other lanes of this same wave.
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (lane < nq && my_k > 0) {
-            const uint32_t* list = nbr + lane * a.lds_stride;
-            write_cov_record(a, my_s, my_k, a.cv.sx[my_s], a.cv.sy[my_s], a.cv.sz[my_s], my_flags,
-                             a.cv.sx, a.cv.sy, a.cv.sz, [&](int l) { return list[l]; });
-            if (my_flags) {
-                const uint32_t slot = atomicAdd(a.out.nflagged, 1u);
-                a.out.flagged[slot] = static_cast<uint32_t>(my_s);
-                atomicAdd(a.out.nflagged + ((my_flags & ST_INCOMPLETE) ? 2 : 1), 1u);
+        if (a.mode == 0) held += nq;
+        const bool last = nq == 0;
+        if (a.mode == 0 && (last || held + static_cast<int>(per) > kRestHeld)) {
+            // The lists were written by other lanes of this same wave.
+            wave_lds_order();
+            if (lane < held && my_k > 0) {
+                const uint32_t* list = nbr + lane * a.lds_stride;
+                write_cov_record(a, my_s, my_k, a.cv.sx[my_s], a.cv.sy[my_s], a.cv.sz[my_s],
+                                 my_flags, a.cv.sx, a.cv.sy, a.cv.sz,
+                                 [&](int l) { return list[l]; });
+                if (my_flags) {
+                    const uint32_t slot = atomicAdd(a.out.nflagged, 1u);
+                    a.out.flagged[slot] = my_s;
+                    atomicAdd(a.out.nflagged + ((my_flags & ST_INCOMPLETE) ? 2 : 1), 1u);
+                }
             }
+            wave_lds_order();
+            held = 0;
+            my_k = 0;
+            my_flags = 0;
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        if (last) break;
+        base = total;
+        if (drawn0 < total) {
+            uint32_t d = 0;
+            if (lane == 0) d = atomicAdd(a.out.nflagged + 5, per);
+            base = drawn0 + lane_u32(d, 0);
+        }
     }
-    if (a.out.counters && lane == 0 && nrows) {
+    if (a.out.counters && lane == 0) {
         atomicAdd(a.out.counters + 0, static_cast<unsigned long long>(cnt[0]));
         atomicAdd(a.out.counters + 1, static_cast<unsigned long long>(cnt[1]));
         atomicAdd(a.out.counters + 2, static_cast<unsigned long long>(cnt[2]));
@@ -2443,11 +2474,11 @@ void launch_knn(const CloudView& cv, const FusedProgram& prog, int mode,
     const GridParams& g = cv.g;
     a.margin = 1e-6 * fmin(g.c, g.cz) +
                1e-15 * (fabs(g.ox) + fabs(g.oy) + fabs(g.oz)) + 1e-300;
-    // The rest: a grid for the few rows usually left (one wave per kRestRows
-    // of them; the kernel walks any number).
-    const uint32_t rest = static_cast<uint32_t>(std::min<uint64_t>(
-        div_up(cv.n, kRestRows), a.all_rows ? 65536u : 8192u));
-    const size_t lds = (kScratchWords + (mode != 0 ? 0 : kRestRows * a.lds_stride)) *
+    // The rest: a grid for the few rows usually left (the waves draw what more
+    // there are).
+    const uint32_t rest = static_cast<uint32_t>(
+        std::min<uint64_t>(div_up(cv.n, kRestRows), kRestWaves));
+    const size_t lds = (kScratchWords + (mode != 0 ? 0 : kRestHeld * a.lds_stride)) *
                        sizeof(uint32_t);
     if (tt) {
         if (!tt->ntasks) return;

@@ -52,3 +52,21 @@ def test_limits(oracle, kind, n, k):
     b.close()
     slow.close()
     c.close()
+
+
+@pytest.mark.parametrize("n", [4, 5, 17, 32767, 32769, 131071, 131072, 131080, 200003])
+def test_growing_search_row_counts(n):
+    # Every row by the growing search, at counts beside the waves' first rows,
+    # the lists held together and the larger draws: the same columns, statuses
+    # and lists as the query-per-lane search.
+    rng = np.random.default_rng(n)
+    x, y, z = np.ascontiguousarray((rng.uniform(0, 1, (n, 3)) * [n ** 0.5, n ** 0.5, 1.0]).T)
+    c, slow = g.Context(0), g.Context(0)
+    slow.set_tuning("set_select", 0)
+    a, b = c.cloud(x, y, z), slow.cloud(x, y, z)
+    k = min(8, n - 1)
+    st = [g.stage(g.STAGE_COVFEAT, k, features=g.F_ALL10)]
+    same_bits(b.run(st, init=np.nan), a.run(st, init=np.nan))
+    assert np.array_equal(a.knn(k)[0], b.knn(k)[0])
+    slow.close()
+    c.close()
