@@ -18,6 +18,8 @@ def cloud(kind, n):
         p = np.tile([1.0, -5.0, 0.0], (n, 1))
     elif kind == "millimetres":  # a fine scan in geocentric coordinates
         p = rng.uniform(0, 1, (n, 3)) * [0.02, 0.02, 0.002] + [5e5, -4e6, -3e6]
+    elif kind == "tall":  # neighbors farther than the search's largest radius
+        p = rng.uniform(0, 1, (n, 3)) * [10.0, 10.0, 1.5 * n]
     elif kind.startswith("scale"):  # spacings at and beyond the FP32 keys' range
         p = rng.normal(size=(n, 3)) * float(kind[5:])
     else:  # "corner": all coordinates large and negative
@@ -33,7 +35,7 @@ def same_bits(a, b):
 
 @pytest.mark.parametrize("k", [1, 8, 9, 20, 36, 40])
 @pytest.mark.parametrize("n", [63, 65, 100, 333])
-@pytest.mark.parametrize("kind", ["coincident", "millimetres", "corner", "scale1e17", "scale1e18",
+@pytest.mark.parametrize("kind", ["coincident", "millimetres", "corner", "tall", "scale1e17", "scale1e18",
                                   "scale1e20", "scale1e40", "scale1e-12", "scale1e-21"])
 def test_limits(oracle, kind, n, k):
     x, y, z = cloud(kind, n)
