@@ -352,9 +352,10 @@ class Context:
         return out.tobytes()
 
     def autotune(self, cloud, stages, factors=(0.4, 0.5, 0.6, 0.75, 0.9)):
-        """Times the run for each column-size factor, then the search's
-        queries per wave; the fastest settings are kept for the cloud's
-        (density, k) bucket.  Returns (factor, ms of the fastest run)."""
+        """Times the run for each column-size factor, then the search's shape
+        (queries per wave and, from 38 entries on, z grouping); the fastest
+        settings are kept for the cloud's (density, k) bucket.  Returns
+        (factor, ms of the fastest run)."""
         stages = list(stages)
         arr = (GfStage * len(stages))(*stages)
         f = np.ascontiguousarray(factors, dtype=np.float64)

@@ -1652,7 +1652,7 @@ int gf_autotune(gf_ctx* ctx, gf_cloud* cloud, const gf_stage* stages, int nstage
         TuneEntry win{};
         try {
             // Coordinate descent: the column-size factor, then the search's
-            // queries per wave.
+            // shape (the z grouping shapes only the wave-per-query search).
             for (int fi = 0; fi < nfactors; ++fi) {
                 if (!(factors[fi] > 0)) throw Error(GF_ERR_ARG, "factors must be positive");
                 c->tune.forced_factor = factors[fi];
@@ -1664,6 +1664,23 @@ int gf_autotune(gf_ctx* ctx, gf_cloud* cloud, const gf_stage* stages, int nstage
             }
             c->tune.forced_factor = bestf;
             win.cell_factor = bestf;
+            const int stride = stages[0].stage == GF_STAGE_NORMAL ? 1 : stages[0].stride;
+            const uint64_t entries = static_cast<uint64_t>(stride) *
+                                     std::min<uint64_t>(n, stage_neighbors(stages[0]));
+            if (entries > kLaneMaxFetch && entries < static_cast<uint64_t>(kMaxFetch)) {
+                int bestgz = saved.group_z;
+                for (int gz : {0, 1, 2, 3, 4}) {
+                    if (gz == saved.group_z) continue;  // measured above
+                    c->tune.group_z = gz;
+                    const double ms = measure();
+                    if (ms < best) {
+                        best = ms;
+                        bestgz = gz;
+                    }
+                }
+                c->tune.group_z = bestgz;
+                win.group_z = bestgz + 1;
+            }
             const int q0 = saved.q_per_wave;
             int bestq = q0;
             for (int q : {16, 32, 64}) {

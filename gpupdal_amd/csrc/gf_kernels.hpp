@@ -122,7 +122,7 @@ struct KnnTuning {
     int32_t ring_max;    // budget before a row is marked incomplete
     int32_t small_col;   // columns up to this size are taken whole
     int32_t group_z;     // wave-per-query search: z cells beyond the first a query group may span
-    int32_t q_per_wave;  // queries per wave (0: by the number of points)
+    int32_t q_per_wave;  // queries per wave (0: 64, and 16 for 38 and more entries)
     int32_t set_select;  // 1: lane-per-query search; 0: every row by the growing search
 };
 
@@ -198,8 +198,10 @@ struct TileTables {
     uint32_t classes;        // knn_class_bit() of every searched tile's capacity, or-ed
 };
 
-// Queries per wave of the search.
+// Queries per wave of the search (a task of a batch).
 constexpr int kQueriesPerWave = 64;
+// The largest result capacity of the query-per-lane search.
+constexpr int kLaneMaxFetch = 37;
 // The search kernel instance that serves a result capacity, as a bit.
 uint32_t knn_class_bit(int fetch);
 

@@ -101,6 +101,8 @@ struct KnnArgs {
     uint32_t ntiles;
     int32_t fetch_lo, fetch_hi;  // tiled: the result capacities this launch serves
     int32_t all_rows;        // k_knn_rest: every row instead of out.deferred
+    int32_t group_q;         // k_knn_group: queries per wave (q_per_wave is a multiple)
+    int32_t group_own;       // k_knn_group: a wave may search its left rows itself
 };
 
 // What a wavefront needs of its cloud or tile: the grid, the column starts,
@@ -1267,7 +1269,15 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
         const float vb = rest ? ex.y * ey.y * ez.y / static_cast<float>(rest) : INFINITY;
         const float v = fminf(va, vb);
         const float r3 = v < INFINITY ? cbrtf(per * v * 0.23873241f) : 0.0f;
-        r_first = fminf(kRadiusFactor * fmaxf(r2, r3), r_cap);
+        const float est = fmaxf(r2, r3);
+        r_first = fminf(kRadiusFactor * est, r_cap);
+        // Where the estimate itself is beyond the largest radius, nearly every
+        // row would be left after all rounds (500k points of a uniform
+        // volume, k 32: 1.0 of 8.6 ms): they are left at once.
+        if (est > r_cap) {
+            defer |= pending;
+            pending = false;
+        }
     }
     uint64_t cnt_pass = 0, cnt_cand = 0, cnt_sort = 0;
     for (int round = 0; round < (kBail ? 2 : 3); ++round) {
@@ -1593,8 +1603,18 @@ void k_knn_pair(KnnArgs a)
 // kLaneMaxFetch entries; its lists and registers grow with them): the
 // wave's queries form groups that share a 2 x 2 block of columns and a short
 // z range, and one candidate box of up to 256 points held in registers; each
-// query's FP64 distances are selected by ballots across the wave.  Rows not
-// certified by that box go to k_knn_rest.
+// query's FP64 distances are selected by ballots across the wave.  Rows whose
+// box holds too many points, or that it does not certify, go to k_knn_rest;
+// but where the latter are most of the wave's and one cloud's launch fills the
+// chip the wave searches them itself, from its groups' half-widths on (such
+// clouds leave rows everywhere, so the waves stay even; tiles of a batch differ:
+// 64 tiles of 20k points, k 16 and 48, 5.4 ms so and 5.0).
+//
+// Search times, ms, with 16 / 32 / 64 queries per wave: 1M points, k 48, 4.6 /
+// 4.8 / 5.1; 60k points, k 48, 0.43 / 0.56 / 0.69; 5k points, k 40, 0.16 / 0.21 /
+// 0.35.  Uncertified rows by the waves themselves and by k_knn_rest: 500k points
+// of a uniform volume, k 48, 6.1 and 7.1; of normal density, k 40, 4.1 and 4.4;
+// 60k points, k 60, where 3750 waves leave the chip half empty, 1.05 and 0.58.
 template <bool kTiled>
 // Four waves per SIMD: the selection is a chain of ballots and LDS round
 // trips, so more resident waves hide more of its latency.
@@ -1602,12 +1622,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 {
     extern __shared__ uint32_t s_lds[];
     const int lane = __lane_id();
-    const int Q = a.q_per_wave;
     WaveGrid wg;
     uint64_t q0;
     int nq;
-    if (!wave_queries<kTiled>(a, xcd_logical_block(blockIdx.x, gridDim.x), Q, wg, q0, nq)) return;
+    // A task's queries, group_q of them to a wave.
+    const uint32_t parts = static_cast<uint32_t>(a.q_per_wave / a.group_q);
+    const uint32_t block = xcd_logical_block(blockIdx.x, gridDim.x);
+    if (!wave_queries<kTiled>(a, block / parts, a.q_per_wave, wg, q0, nq)) return;
     if (kTiled && (wg.fetch > a.fetch_hi || wg.fetch < a.fetch_lo)) return;
+    const int first = static_cast<int>(block % parts) * a.group_q;
+    if (nq <= first) return;
+    q0 += first;
+    nq = min(nq - first, a.group_q);
     const CloudView& cv = a.cv;
     const GridParams& g = wg.g;
     const int fetch = wg.fetch;
@@ -1620,6 +1646,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 
     uint8_t my_flags = 0;
     uint64_t left = 0;  // the wave's queries not settled here
+    int my_ring = 1;    // the first box of the lane's query if it is left
     uint64_t cnt[3] = {0, 0, 0};  // search passes, candidates, selections
     int qi = 0;
     int rg_prev = 1;  // box half-width of the previous group (density guess)
@@ -1818,9 +1845,31 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
                     if (done) finish_query(a, wg, best, false, s, qslot, lane, nbr, my_flags);
                 }
             }
-            if (!done) left |= 1ull << qslot;
+            if (!done) {
+                left |= 1ull << qslot;
+                if (lane == qslot) my_ring = cached ? rg + 1 : 1;
+            }
         }
         qi += gm;
+    }
+    const uint64_t own = a.group_own ? left & __ballot(my_ring > 1) : 0ull;
+    if (2 * __popcll(own) > nq) {
+        for (uint64_t m = own; m; m &= m - 1) {
+            const int qslot = __builtin_ctzll(m);
+            const double qx = lane_value(wx, qslot), qy = lane_value(wy, qslot),
+                         qz = lane_value(wz, qslot);
+            const int qcx = static_cast<int>(cell_coord(qx, g.ox, g.inv_c, g.gx));
+            const int qcy = static_cast<int>(cell_coord(qy, g.oy, g.inv_c, g.gy));
+            const int qcz = static_cast<int>(cell_coord(qz, g.oz, g.inv_cz, g.gz));
+            Ent best;
+            bool incomplete = false;
+            search_single(a, wg, qx, qy, qz, qcx, qcy, qcz,
+                          min(static_cast<int>(lane_u32(static_cast<uint32_t>(my_ring), qslot)),
+                              a.tune.ring_max),
+                          lane, scratch, best, incomplete, cnt);
+            finish_query(a, wg, best, incomplete, q0 + qslot, qslot, lane, nbr, my_flags);
+        }
+        left &= ~own;
     }
     if (left) {
         uint32_t at = 0;
@@ -1850,7 +1899,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     if (my_flags) {
         const uint32_t slot = atomicAdd(a.out.nflagged, 1u);
         a.out.flagged[slot] = static_cast<uint32_t>(s);
-        atomicAdd(a.out.nflagged + 1, 1u);
+        atomicAdd(a.out.nflagged + ((my_flags & ST_INCOMPLETE) ? 2 : 1), 1u);
     }
 }
 
@@ -1931,8 +1980,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
             const int qcz = uniform_i32(static_cast<int>(cell_coord(qz, g.oz, g.inv_cz, g.gz)));
             Ent best;
             bool incomplete = false;
-            search_single(a, wg, qx, qy, qz, qcx, qcy, qcz, first_ring(a, wg, qcx, qcy, qcz, lane),
-                          lane, scratch, best, incomplete, cnt);
+            // (what k_knn_group leaves is mostly too dense for it: one ring
+            // first; 500k points of normal density, k 40, 4.1 ms against 5.0)
+            const int ring = wg.fetch > kLaneMaxFetch ? a.tune.ring0
+                                                      : first_ring(a, wg, qcx, qcy, qcz, lane);
+            search_single(a, wg, qx, qy, qz, qcx, qcy, qcz, ring, lane, scratch, best, incomplete,
+                          cnt);
             finish_query(a, wg, best, incomplete, s, held + p, lane, nbr, my_flags);
             if (lane == held + p) {
                 my_s = s;
@@ -2418,7 +2471,8 @@ __global__ __launch_bounds__(256) void k_eigen_batch(const double* __restrict__ 
 // entries of the query-per-lane instances follow it; above kLaneMaxFetch
 // their registers would not leave two waves per SIMD, and the wave-per-query
 // search serves.
-constexpr int kLaneMaxFetch = 37;
+constexpr int kGroupQueries = 16;           // k_knn_group's queries per wave
+constexpr uint32_t kGroupOwnWaves = 16384;  // four rounds of the waves that fit the chip
 
 static int lane_class(int fetch)
 {
@@ -2449,9 +2503,11 @@ static void launch_lane(KnnArgs& a, uint32_t classes, uint32_t blocks, hipStream
     if (classes & 8u) {
         a.fetch_lo = kLaneMaxFetch + 1;
         a.fetch_hi = kMaxFetch - 1;
-        const size_t lds = (kScratchWords + (a.mode != 0 ? 0 : a.q_per_wave * a.lds_stride)) *
+        const size_t lds = (kScratchWords + (a.mode != 0 ? 0 : a.group_q * a.lds_stride)) *
                            sizeof(uint32_t);
-        hipLaunchKernelGGL(k_knn_group<kTiled>, dim3(blocks), dim3(64), lds, s, a);
+        const uint32_t waves = blocks * static_cast<uint32_t>(a.q_per_wave / a.group_q);
+        a.group_own = !kTiled && waves >= kGroupOwnWaves;
+        hipLaunchKernelGGL(k_knn_group<kTiled>, dim3(waves), dim3(64), lds, s, a);
     }
 }
 
@@ -2470,6 +2526,7 @@ void launch_knn(const CloudView& cv, const FusedProgram& prog, int mode,
     const int max_k = tt ? tt->max_k : prog.k;
     a.q_per_wave = tt ? tt->q_per_wave
                       : (tune.q_per_wave > 0 ? tune.q_per_wave : kQueriesPerWave);
+    a.group_q = tune.q_per_wave > 0 ? a.q_per_wave : kGroupQueries;
     a.lds_stride = max_k | 1;  // odd stride: lanes hit distinct LDS banks
     const GridParams& g = cv.g;
     a.margin = 1e-6 * fmin(g.c, g.cz) +

@@ -152,9 +152,10 @@ int gf_set_tuning(gf_ctx *ctx, const char *key, double value);
  *      (makeKnnGridConfig / makeAdaptiveKnnConfig, src/index/SpatialIndex.cpp
  *      :434-631).  gf_autotune times the whole run over a cloud for each
  *      candidate column-size factor (column edge = factor * sqrt(k / (pi *
- *      2-D density))), keeps the fastest, then tries the search's queries
- *      per wave (16, 32, 64), keeping a change that is faster, and stores the
- *      result for the cloud's (density, k) bucket.  Later grids in that bucket
+ *      2-D density))), keeps the fastest, then tries the search's shape --
+ *      z cells a query group spans (0..4; result capacities of 38 to 63 only)
+ *      and queries per wave (16, 32, 64) -- keeping each change that is
+ *      faster, and stores the result for the cloud's (density, k) bucket.  Later grids in that bucket
  *      (clouds and batch tiles) use its factor; clouds use its shape, and a
  *      batch's search launches the shape of its largest tile's bucket.  No
  *      row's result depends on any of them.  The table is saved and loaded as

@@ -72,3 +72,36 @@ def test_growing_search_row_counts(n):
     assert np.array_equal(a.knn(k)[0], b.knn(k)[0])
     slow.close()
     c.close()
+
+
+@pytest.mark.parametrize("n", [262080, 262144, 262209])
+@pytest.mark.parametrize("kind", ["volume", "normal"])
+def test_waves_searching_their_own_rows(kind, n):
+    # The wave-per-query search beside the launch size from which its waves
+    # search most of their uncertified rows themselves.
+    rng = np.random.default_rng(n)
+    p = rng.uniform(0, 50.0, (n, 3)) if kind == "volume" else rng.normal(size=(n, 3)) * [90, 90, 5]
+    x, y, z = np.ascontiguousarray(p.T)
+    c, slow = g.Context(0), g.Context(0)
+    slow.set_tuning("set_select", 0)
+    a, b = c.cloud(x, y, z), slow.cloud(x, y, z)
+    st = [g.stage(g.STAGE_EIGENVALUES, 39)]
+    same_bits(b.run(st, init=np.nan), a.run(st, init=np.nan))
+    assert np.array_equal(a.knn(38)[0], b.knn(38)[0])
+    slow.close()
+    c.close()
+
+
+def test_autotuner_tries_the_z_grouping(tmp_path):
+    # From 38 entries on the z grouping shapes the search, and is tuned.
+    c = g.Context(0)
+    rng = np.random.default_rng(5)
+    cl = c.cloud(*np.ascontiguousarray((rng.uniform(0, 40, (20000, 3)) * [1, 1, 0.1]).T))
+    for knn, tuned in ((39, True), (16, False)):
+        c.autotune(cl, [g.stage(g.STAGE_COVFEAT, knn)], factors=(0.6,))
+        c.save_tuning(tmp_path / "t")
+        rows = [r.split() for r in (tmp_path / "t").read_text().splitlines() if r[0] != "#"]
+        assert any((int(r[3]) > 0) == tuned for r in rows), (knn, rows)
+        if tuned:
+            assert all(int(r[3]) > 0 for r in rows)
+    c.close()
