@@ -1600,7 +1600,8 @@ void k_knn_pair(KnnArgs a)
 // ------------------------------------------------- wave-per-query search --
 //
 // Neighborhoods too large for the query-per-lane search (more than
-// kLaneMaxFetch entries; its lists and registers grow with them): the
+// kLaneMaxFetch entries; its lists and registers grow with them), and those of
+// 22 entries and more on small clouds: the
 // wave's queries form groups that share a 2 x 2 block of columns and a short
 // z range, and one candidate box of up to 256 points held in registers; each
 // query's FP64 distances are selected by ballots across the wave.  Rows whose
@@ -2470,8 +2471,15 @@ __global__ __launch_bounds__(256) void k_eigen_batch(const double* __restrict__ 
 // The search kernels that serve a result capacity.  List entries and kept
 // entries of the query-per-lane instances follow it; above kLaneMaxFetch
 // their registers would not leave two waves per SIMD, and the wave-per-query
-// search serves.
+// search serves.  So it does for 22 entries and more on clouds (or batches) of
+// fewer than kWideMin points: the largest instance's waves, 64 queries each, are
+// few and long there.  Search, ms, by that instance and wave per query: 3k
+// points in dense balls, k 36, 0.50 and 0.20; 60k airborne points, k 31, 0.62
+// and 0.34; 125k, k 36, 0.80 and 0.59.  At 131,072 points the exact tree is built
+// beside the search, and finds fewer free slots beside the wave-per-query
+// kernel: 200k, k 36, search 1.28 and 0.94, but the call 1.90 and 2.05.
 constexpr int kGroupQueries = 16;           // k_knn_group's queries per wave
+constexpr uint64_t kWideMin = 131072;
 constexpr uint32_t kGroupOwnWaves = 16384;  // four rounds of the waves that fit the chip
 
 static int lane_class(int fetch)
@@ -2484,6 +2492,11 @@ uint32_t knn_class_bit(int fetch) { return 1u << lane_class(fetch); }
 template <bool kTiled>
 static void launch_lane(KnnArgs& a, uint32_t classes, uint32_t blocks, hipStream_t s)
 {
+    int group_lo = kLaneMaxFetch + 1;
+    if (a.cv.n < kWideMin && (classes & 4u)) {
+        classes = (classes & ~4u) | 8u;
+        group_lo = 22;
+    }
     bool again = false;
     auto one = [&](uint32_t bit, int lo, int hi, auto lane, auto pair) {
         if (!(classes & bit)) return;
@@ -2501,7 +2514,7 @@ static void launch_lane(KnnArgs& a, uint32_t classes, uint32_t blocks, hipStream
     one(2u, 10, 21, k_knn_lane<40, 24, 2, kTiled>, k_knn_pair<32, 24, 2, kTiled>);
     one(4u, 22, kLaneMaxFetch, k_knn_lane<56, 40, 2, kTiled>, k_knn_pair<48, 40, 2, kTiled>);
     if (classes & 8u) {
-        a.fetch_lo = kLaneMaxFetch + 1;
+        a.fetch_lo = group_lo;
         a.fetch_hi = kMaxFetch - 1;
         const size_t lds = (kScratchWords + (a.mode != 0 ? 0 : a.group_q * a.lds_stride)) *
                            sizeof(uint32_t);

@@ -8,6 +8,7 @@ import pytest
 
 import gpupdal_amd as g
 from helpers import set_equal_rows
+from test_gpu_search_paths import cloud as path_cloud
 
 pytestmark = pytest.mark.gpu
 
@@ -104,4 +105,37 @@ def test_autotuner_tries_the_z_grouping(tmp_path):
         assert any((int(r[3]) > 0) == tuned for r in rows), (knn, rows)
         if tuned:
             assert all(int(r[3]) > 0 for r in rows)
+    c.close()
+
+
+# 22 to 37 entries are searched by the query-per-lane search from 131,072
+# points (of a cloud or batch) on: copies of a cloud side by side, beside that
+# count, at the instance's limits.
+@pytest.mark.parametrize("n", [131071, 131072, 131137])
+@pytest.mark.parametrize("k", [22, 36, 37])
+@pytest.mark.parametrize("kind", ["ragged", "clumps", "shells", "tower"])
+def test_wide_neighborhoods_of_large_clouds(oracle, kind, k, n):
+    p = np.array(path_cloud(kind)).T
+    m = -(-n // len(p))
+    p = np.concatenate([p + [5000.0 * i, 0.0, 0.0] for i in range(m)])[:n]
+    x, y, z = np.ascontiguousarray(p.T)
+    c, slow = g.Context(0), g.Context(0)
+    slow.set_tuning("set_select", 0)
+    cl = c.cloud(x, y, z)
+    st = [g.stage(g.STAGE_COVFEAT, k - 1)]
+    want = slow.cloud(x, y, z).run(st, init=np.nan)
+    same_bits(cl.run(st, init=np.nan), want)
+    if n == 131072:
+        tree = oracle.kd3(x, y, z)
+        assert set_equal_rows(cl.knn(k)[0], tree.neighbors_all(k, threads=8)).all()
+    # The same points as a batch of two tiles.
+    half = n // 2
+    tiles = [(x[:half], y[:half], z[:half]), (x[half:], y[half:], z[half:])]
+    b = c.batch(tiles)
+    got = b.run(st, init=np.nan)
+    for t in (0, 1):
+        alone = slow.cloud(*tiles[t]).run(st, init=np.nan)
+        same_bits(([[b.tile(col, t) for col in got[0][0]]], [b.tile(got[1][0], t)]), alone)
+    b.close()
+    slow.close()
     c.close()
