@@ -39,19 +39,21 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 # Algorithmic bytes per point of the search (k_knn_lane and the kernels for
-# the rows it leaves): the query's FP64 xyz (24 B) and grid key (4 B) read once, its covariance record written (one
-# 64-byte record: six FP64 entries, the row-flags word and one pad word).
+# the rows it leaves): the query's FP64 xyz (24 B) and grid key (4 B) read
+# once, its covariance record written (one 64-byte record: six FP64 entries,
+# the row-flags word and one pad word).
 SEARCH_BYTES_PER_POINT = 92.0
-# HBM traffic of one k_knn launch on the bench workload (4,000,000 points,
-# knn=16), from rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE runs of this
-# script (KiB per dispatch), each scaled by the same counter on a 1 GiB copy
-# kernel in the same runs: FETCH_SIZE reads 0.5 of the copied bytes there
-# (factor 2.0), WRITE_SIZE 1.0 (factor 1.0).  kernel_commit names the commit
-# whose k_knn source the counters were taken on; the runs, commands and raw
-# counter values are in profiles/k_knn_plain_4M_knn16_traffic.md.
-MEASURED_TRAFFIC = {"points": 4_000_000, "knn": 16, "fetch_kib": 83510.1,
-                    "write_kib": 312652.9, "fetch_factor": 2.0, "write_factor": 1.0,
-                    "kernel_commit": "6472501"}
+# HBM traffic of one search (k_knn_lane + k_knn_pair + k_knn_rest) on the bench
+# workload (4,000,000 points, knn=16), from rocprofv3 --pmc FETCH_SIZE and --pmc
+# WRITE_SIZE runs of this script (KiB per dispatch, the three kernels added),
+# each scaled by the same counter on a 1 GiB copy kernel in the same runs:
+# FETCH_SIZE reads 0.5 of the copied bytes there (factor 2.0), WRITE_SIZE 1.0
+# (factor 1.0).  kernel_commit names the commit whose search the counters were
+# taken on; the runs, commands and raw counter values are in
+# profiles/search_plain_4M_knn16_traffic.md.
+MEASURED_TRAFFIC = {"points": 4_000_000, "knn": 16, "fetch_kib": 1781158.9,
+                    "write_kib": 268287.8, "fetch_factor": 2.0, "write_factor": 1.0,
+                    "kernel_commit": "3924b78"}
 # FP64 flops per candidate distance: 3 sub, 3 mul, 2 add.
 FLOPS_PER_CANDIDATE = 8.0
 HBM_PEAK_GBS = 8000.0
@@ -139,7 +141,7 @@ def gpu_leg(args):
         roofline={"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                   "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                   "traffic_source": (None if traffic is None else
-                                     "rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated; k_knn as of "
+                                     "rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated; search as of "
                                      "commit " + mt["kernel_commit"]),
                   "kernel": "k_knn_lane + k_knn_pair + k_knn_rest (kNN search + FP64 covariance)",
                   "bytes_per_point": SEARCH_BYTES_PER_POINT,

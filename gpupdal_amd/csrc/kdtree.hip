@@ -885,8 +885,8 @@ __global__ __launch_bounds__(kLvlThreads) void k_kd_big_minmax(
 //
 // Bound by the latency of the passes over one node.  With every node above the
 // subtree size (2048) split by device-wide levels the runs that wait for the
-// tree took, ms: 48k points 1.88, 250k 2.18, 4M 8.7; with this 1.62, 1.56, 7.7.
-// kMid and threads (250k / 4M points, ms): 8192 and 256 2.08 / 8.2 (more
+// tree take, ms: 48k points 2.01, 250k 2.21, 4M 8.2; with this 1.74, 1.67, 7.5.
+// kMid and threads (250k / 4M points, ms, in runs with an earlier search): 8192 and 256 2.08 / 8.2 (more
 // levels), 16384 and 256 1.58 / 8.0, and 1024 1.48 / 8.3 (workgroups wait for
 // the search's to drain), 32768 and 512 1.56 / 7.7.
 constexpr uint32_t kMid = 32768;

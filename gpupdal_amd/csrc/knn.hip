@@ -1,18 +1,20 @@
-// knn.hip -- wavefront-per-query k-nearest-neighbor search over the column
-// grid, fused with the neighborhood covariance; plus the per-row eigensolve
-// and stage-output kernel.
+// knn.hip -- k-nearest-neighbor and radius search over the column grid, fused
+// with the neighborhood covariance; plus the per-row eigensolve and
+// stage-output kernel.
 //
 // Replaces the reference's thread-per-query knnGatherKernel with its fused
 // covariance, the device eigen kernel and the projection kernels
 // (src/index/SpatialIndexKernels.cu:716-1086, 1716-1769;
 // src/stages/NeighborhoodKernels.cu:67-119, 422-485).
 //
-// Two kernels share the work: k_knn_lane searches up to 64 consecutive sorted
-// queries per wave, one per lane, over one shared candidate box (see there);
-// k_knn_rest searches the few rows that leaves, one per wave, with a box that
-// grows around the row's own cell.  Both find the fetch + 1 smallest (d2,
-// point id) pairs with the FP64 squared distances KD3Index computes (d0*d0 +
-// d1*d1 + d2*d2, left to right, no FMA).
+// Four kernels share the work.  k_knn_lane searches 64 queries per wave, one per
+// lane, over one shared box of points staged in LDS; k_knn_pair the groups it
+// finds too crowded, half a group at a time with two lanes per query.
+// k_knn_group serves larger neighborhoods (and middling ones of small clouds)
+// with one wave per query.  k_knn_rest searches the rows these leave, one per
+// wave, with a box that grows around the row's own cell.  All find the fetch + 1
+// smallest (d2, point id) pairs with the FP64 squared distances KD3Index
+// computes (d0*d0 + d1*d1 + d2*d2, left to right, no FMA).
 //
 // Certification.  A query's list is exact when its fetch-th distance is below
 // the distance from the query to the nearest face of the examined region
@@ -24,7 +26,7 @@
 //
 // Covariance.  A row's FP64 covariance (two-pass mean) is formed by one lane
 // from the kept list in (d2, id) order, the same sums in the same order in
-// both kernels, and written in sorted order for the eigen/feature kernel.
+// every kernel, and written in sorted order for the eigen/feature kernel.
 #include "gf_eigen.hpp"
 #include "gf_internal.hpp"
 #include "gf_kernels.hpp"
@@ -874,18 +876,18 @@ __device__ __forceinline__ bool wave_queries(const KnnArgs& a, uint64_t task, in
 // A few lanes not final go to k_knn_rest; more of them are tried again with
 // a larger radius first.
 //
-// Bound by vector instructions (staging, walks and the sorting network) at two
-// waves per SIMD.  Against the wave-per-query search (k_knn_group) for every
-// row, search time: 4M points k 16 8.4 -> 5.4 ms, 777k k 8 stride 3 3.6 ->
-// 2.2, 250k k 10 1.67 -> 0.64; 10M points of terrain and flat roofs, k 32,
-// 34 -> 32.
+// Bound by vector instructions (staging, walks and the sorting network) at the
+// five to seven waves per CU that their LDS allows (22.0, 26.0 and 30.0 KB by
+// instance), so that some SIMDs hold two: hence at most 256 registers.  Against
+// the wave-per-query search for every row, search time: 4M points k 16 8.4 -> 5.2
+// ms, 777k k 8 stride 3 3.6 -> 2.2, 250k k 10 1.67 -> 0.63; 10M points of terrain
+// and flat roofs, k 32, 34 -> 27.
 constexpr int kLaneSlack = 2;   // entries beyond fetch + 1 put in exact order
 // First radius over the one the density's estimate gives, and the points a
 // lane's radius should hold over fetch + 1 (measured best of 1.2 to 1.7 and 1.5
 // to 2.1: smaller ones fail lanes, larger ones fill boxes and lists).
 constexpr float kRadiusFactor = 1.35f;
 constexpr float kListFactor = 1.8f;
-constexpr int kLaneTries = 3;   // radii tried per query
 constexpr int kLaneFew = 6;     // lanes not worth another round of their own
 constexpr uint32_t kStageMax = 512;    // points staged per round
 constexpr int kStageSlots = 16;        // points of the box's columns per lane and round
@@ -1528,7 +1530,7 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
             ++tries;
             const float f = sqrtf(1.5f * static_cast<float>(fetch) /
                                   static_cast<float>(max(cnt, 1u)));
-            const bool give_up = few || in_ball || tries >= kLaneTries || rl >= r_cap;
+            const bool give_up = few || in_ball || rl >= r_cap;
             r_need = rl * fminf(fmaxf(f, 1.3f), 2.0f);
             defer |= give_up;
             pending = !give_up;
@@ -1537,7 +1539,9 @@ __device__ __forceinline__ bool search_group(const KnnArgs& a, const WaveGrid& w
         }
         wave_lds_order();  // the next round stages over this one's box
     }
-    defer |= pending;  // not reached: every round settles or counts a try of a lane
+    // Lanes still pending: their last round failed, or its box was halved
+    // without them.
+    defer |= pending;
     defer = defer && part == 0;
     const uint64_t dm = __ballot(defer);
     if (dm) {
@@ -2469,9 +2473,10 @@ __global__ __launch_bounds__(256) void k_eigen_batch(const double* __restrict__ 
 } // namespace
 
 // The search kernels that serve a result capacity.  List entries and kept
-// entries of the query-per-lane instances follow it; above kLaneMaxFetch
-// their registers would not leave two waves per SIMD, and the wave-per-query
-// search serves.  So it does for 22 entries and more on clouds (or batches) of
+// entries of the query-per-lane instances follow it, and with them LDS and
+// registers: 150, 222 and, at 37 entries, already more than the 256 that are left
+// (42 to 90 spilled).  Above kLaneMaxFetch the wave-per-query search serves.  So
+// it does for 22 entries and more on clouds (or batches) of
 // fewer than kWideMin points: the largest instance's waves, 64 queries each, are
 // few and long there.  Search, ms, by that instance and wave per query: 3k
 // points in dense balls, k 36, 0.50 and 0.20; 60k airborne points, k 31, 0.62

@@ -163,7 +163,8 @@ int gf_set_tuning(gf_ctx *ctx, const char *key, double value);
  *      q_per_wave knn_waves, 0 = the context's setting; three-field lines are
  *      read as factor only).  The same knobs can be set for a context with
  *      gf_set_tuning ("group_z": query grouping of the search for 38 and more
- *      entries, "q_per_wave", and "knn_waves", which has no effect). */
+ *      entries (22 and more on small clouds), "q_per_wave", and "knn_waves",
+ *      which has no effect). */
 int gf_autotune(gf_ctx *ctx, gf_cloud *cloud, const gf_stage *stages, int nstages,
                 const double *factors, int nfactors, double *best_factor, double *best_ms);
 int gf_tuning_save(gf_ctx *ctx, const char *path);

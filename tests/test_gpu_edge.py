@@ -242,11 +242,11 @@ def _bits_equal(a, b):
 
 @pytest.mark.parametrize("cloud", ["dups", "lattice", "dense"])
 def test_set_selection_equals_sorting(ctx, cloud):
-    # Feature neighborhoods with stride 1 are kept as sets, found by the
-    # exact-count threshold selection; switching it off (set_select=0) runs
-    # the sorting selection that lists use.  Every status bit and every
-    # column bit must agree: the same sets, summed in the same (d2, id)
-    # order, flagged (ties, uncertified rows) the same way.
+    # The query-per-lane search (knn 8 and 16) and the wave-per-query search
+    # with its exact-count threshold selection (knn 32 on clouds of this size)
+    # against every row by its own growing search (set_select=0).  Every
+    # status bit and every column bit must agree: the same sets, summed in the
+    # same (d2, id) order, flagged (ties, uncertified rows) the same way.
     if cloud == "dups":
         x, y, z = small_cloud(60000, seed=73, dup_frac=0.03)
     elif cloud == "lattice":
