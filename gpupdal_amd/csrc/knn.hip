@@ -2476,15 +2476,16 @@ __global__ __launch_bounds__(256) void k_eigen_batch(const double* __restrict__ 
 // entries of the query-per-lane instances follow it, and with them LDS and
 // registers: 150, 222 and, at 37 entries, already more than the 256 that are left
 // (42 to 90 spilled).  Above kLaneMaxFetch the wave-per-query search serves.  So
-// it does for 22 entries and more on clouds (or batches) of
-// fewer than kWideMin points: the largest instance's waves, 64 queries each, are
-// few and long there.  Search, ms, by that instance and wave per query: 3k
+// it does for 22 entries and more on clouds (or batches) of fewer than kWideMin
+// points: the largest instance's waves, 64 queries each, are few and long there.  Search, ms, by that instance and wave per query: 3k
 // points in dense balls, k 36, 0.50 and 0.20; 60k airborne points, k 31, 0.62
 // and 0.34; 125k, k 36, 0.80 and 0.59.  At 131,072 points the exact tree is built
 // beside the search, and finds fewer free slots beside the wave-per-query
 // kernel: 200k, k 36, search 1.28 and 0.94, but the call 1.90 and 2.05.
 constexpr int kGroupQueries = 16;           // k_knn_group's queries per wave
+constexpr uint32_t kGroupMaxTasks = 1u << 24;  // tasks of 64 queries cut into waves of 16
 constexpr uint64_t kWideMin = 131072;
+static_assert(uint64_t{kGroupMaxTasks} * (kQueriesPerWave / kGroupQueries) * 64 <= 1ull << 32);
 constexpr uint32_t kGroupOwnWaves = 16384;  // four rounds of the waves that fit the chip
 
 static int lane_class(int fetch)
@@ -2519,6 +2520,8 @@ static void launch_lane(KnnArgs& a, uint32_t classes, uint32_t blocks, hipStream
     one(2u, 10, 21, k_knn_lane<40, 24, 2, kTiled>, k_knn_pair<32, 24, 2, kTiled>);
     one(4u, 22, kLaneMaxFetch, k_knn_lane<56, 40, 2, kTiled>, k_knn_pair<48, 40, 2, kTiled>);
     if (classes & 8u) {
+        // (a launch holds fewer than 2^32 threads)
+        if (blocks >= kGroupMaxTasks) a.group_q = a.q_per_wave;
         a.fetch_lo = group_lo;
         a.fetch_hi = kMaxFetch - 1;
         const size_t lds = (kScratchWords + (a.mode != 0 ? 0 : a.group_q * a.lds_stride)) *
